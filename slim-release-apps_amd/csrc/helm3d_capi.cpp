@@ -793,12 +793,8 @@ int helm3d_set_model(helm3d_ctx* c, const int n[3], const double h[3], const int
     const size_t esz = c->wnc ? 2 : 1;
     CHK(ensure(&c->wn64, &c->wn64_cap, size_t(N) * esz * sizeof(double)));
     CHK(ensure(&c->wn32, &c->wn32_cap, size_t(N) * esz * sizeof(float)));
-    HIPCHK(hipMemcpyAsync(c->wn64, wn_dev, size_t(N) * esz * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-    if (c->wnc)
-        HIPCHK((launch_axpby<double, float>(1.0, 0.0, static_cast<const cpx<double>*>(c->wn64), 0.0, 0.0,
-                                            static_cast<cpx<float>*>(c->wn32), N, false, c->stream)));
-    else
-        HIPCHK(launch_cast_real(static_cast<const double*>(c->wn64), static_cast<float*>(c->wn32), N, c->stream));
+    HIPCHK(launch_copy_cast(static_cast<const double*>(wn_dev), static_cast<double*>(c->wn64),
+                            static_cast<float*>(c->wn32), N * long(esz), c->stream));
 
     fill_opdesc(c->op64, n, c->hc, c->tab64, off, c->wn64, c->wnc, ilo, ihi);
     fill_opdesc(c->op32, n, c->hc, c->tab32, off, c->wn32, c->wnc, ilo, ihi);

