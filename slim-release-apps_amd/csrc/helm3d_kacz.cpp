@@ -11,14 +11,14 @@
 
 namespace helm3d {
 hipError_t launch_kacz_sweep(bool adj, const OpDesc<double>& op, double omega, cpx<double>* x,
-                             const cpx<double>* b, hipStream_t s);
+                             const cpx<double>* b, int nsweeps, hipStream_t s);
 }
 
 namespace {
 
 int sweep(helm3d_ctx* c, int mode, double omega, cpx<double>* x, const cpx<double>* b, int n)
 {
-    for (int s = 0; s < n; ++s) HIPCHK(launch_kacz_sweep(mode != 1, c->op64, omega, x, b, c->stream));
+    HIPCHK(launch_kacz_sweep(mode != 1, c->op64, omega, x, b, n, c->stream));
     return HELM3D_OK;
 }
 

@@ -182,3 +182,25 @@ def test_crmn_matches_oracle(mode):
     r = b - O.hmvp(v, wn, h3, cfg.nt, p6, x)
     rel = np.linalg.norm(r) / np.linalg.norm(b)
     assert abs(rel - info.relres) <= 1e-9 + 1e-6 * rel
+
+
+# The line form of the sweep: blocks of one wave, several waves, the most
+# threads a block takes (rows looped), and either side of the longest line it
+# holds in LDS (299 points forward, 449 adjoint, 224 forward with complex wn).
+LINES = [(3, 4, 3), (47, 4, 5), (49, 3, 4), (224, 4, 3), (225, 3, 4), (299, 4, 4), (300, 4, 4), (385, 3, 3),
+         (449, 4, 3), (450, 4, 3)]
+
+
+@pytest.mark.parametrize("n", LINES, ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("variant", ["forw", "adj", "forw_wnc", "adj_wnc"])
+def test_device_sweep_line_lengths(n, variant):
+    import torch
+    from helm3d import Helm3d
+    npml, h = np.array([[2, 1, 1], [1, 1, 2]]), (10.0, 11.0, 9.0)
+    wn, x, b = _inputs(n, 70 + n[0], variant.endswith("wnc"))
+    print(f"sweep lines n={n} variant={variant}", flush=True)
+    H = Helm3d(n, h, npml, torch.from_numpy(wn).cuda())
+    mode = 2 if variant.startswith("adj") else 1
+    y = H.kacz_sweep(torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda(), mode=mode, nsweeps=2).cpu().numpy()
+    yo = O.kacz_sweep(variant, wn, h, n, npml, 1.5, O.kacz_sweep(variant, wn, h, n, npml, 1.5, x, b), b)
+    assert relerr(y, yo) <= 1e-12
