@@ -8,6 +8,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "bicgstab.hpp"
@@ -141,7 +142,10 @@ struct helm3d_ctx {
     size_t wn32_cap = 0;
     OpDesc<double> op64{};
     OpDesc<float> op32{};
-    StencilGrid grid{};
+    // launch shape per precision: by rule until set_launch or autotune chooses
+    // one shape for both
+    StencilGrid grid{}, grid32{};
+    bool grid_auto = true;
 
     double* part = nullptr;
     size_t part_cap = 0;
@@ -263,6 +267,13 @@ void fill_opdesc(OpDesc<R>& op, const int n[3], const HConst& k, const cpx<R>* t
     }
 }
 
+template <typename R>
+inline const StencilGrid& grid_of(const helm3d_ctx* c)
+{
+    if constexpr (std::is_same<R, double>::value) return c->grid;
+    else return c->grid32;
+}
+
 inline int bind(helm3d_ctx* c)
 {
     if (!c) return fail(HELM3D_ERR_ARG, "null context");
@@ -315,7 +326,7 @@ constexpr long kMaxDeviceCycles = 16;
 // mirror) and the stencil's write-only sink.
 inline int ensure_work(helm3d_ctx* c)
 {
-    const size_t nblk = std::max<size_t>(c->grid.blocks, kMaxPartials);
+    const size_t nblk = std::max<size_t>(std::max(c->grid.blocks, c->grid32.blocks), kMaxPartials);
     CHK(ensure_t(&c->part, &c->part_cap, nblk * 2 * kMaxBasis));
     CHK(ensure_t(&c->small, &c->small_cap, 2 * kMaxBasis + 8));
     CHK(ensure(&c->sink, &c->sink_cap, size_t(kSinkSlots) * sizeof(cpx<double>)));

@@ -57,8 +57,25 @@ struct StencilGrid {
     int tiles_x, tiles_y, kchunk, nchunks, blocks, ty, pf, ry;
 };
 
-// kchunk <= 0 picks a chunk giving ~480 blocks; ty in {4, 8}; pf in 1..4;
-// ry in {1, 2} (2 needs ty = 8; otherwise 1 is used).
+// z planes per block (even) for a launch over columns of `tiles[i]` tiles and
+// nz[i] planes, i < n.  A block marches its planes and two halo planes, blocks
+// run `slots` at a time, and the launch ends with a tail in which slots idle,
+// longer when the last round is nearly empty:
+//   cost(kc) = planes(kc) / slots + (kc + 2) (0.2 + 0.15 (ceil(x) - x)),
+//   planes = sum tiles (nz + 2 chunks), x = blocks / slots,
+// fitted to launches of chunks from 2 planes to the whole column on single
+// grids of 48 x 48 x 40 to 296 x 296 x 168 and on batches of 2 to 8 of them;
+// the chunk it picks is within 5 % of the best of the sweep on each
+// (complex128 48 x 48 x 40: 2 planes 5.7 us, 8 planes 9.8; 84^3: 8 planes 14.6,
+// 6 planes 15.8, 42 planes 34.9; complex64 240 x 240 x 140: 18 planes 47.9, 70
+// planes 58.8; six uneven grids together: 16 planes 13.7 ms, 8 planes 15.1).
+// About two complex128 blocks of 256 threads fit a compute unit, four
+// complex64 ones.
+int stencil_chunk(const long* tiles, const int* nz, int n, int slots);
+constexpr int kSlots64 = 512, kSlots32 = 1024;
+
+// kchunk <= 0 picks the chunk by stencil_chunk for precision R; ty in {4, 8};
+// pf in 1..4; ry in {1, 2} (2 needs ty = 8; otherwise 1 is used).
 template <typename R>
 StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 4, int pf = 2, int ry = 1);
 

@@ -25,6 +25,8 @@
 // computed, so HBM latency overlaps the march.  Block
 // ids are remapped so consecutive tiles of the same chunk land on the same XCD
 // and share halo lines in its L2.
+#include <cmath>
+
 #include "helm27_body.hpp"
 
 namespace helm3d {
@@ -39,6 +41,30 @@ __global__ __launch_bounds__(TX* TY / RY) void helm27_kernel(StencilLaunch<R> L)
 
 }  // namespace
 
+int stencil_chunk(const long* tiles, const int* nz, int n, int slots)
+{
+    int top = 1;
+    for (int i = 0; i < n; ++i) top = std::max(top, nz[i]);
+    top = std::min(top, kMaxChunk);
+    int best = top;
+    double best_cost = 1e300;
+    for (int kc = 2; kc < top + 2; kc += 2) {
+        double blocks = 0.0, planes = 0.0;
+        for (int i = 0; i < n; ++i) {
+            const int ch = (nz[i] + kc - 1) / kc;
+            blocks += double(tiles[i]) * ch;
+            planes += double(tiles[i]) * (nz[i] + 2 * ch);
+        }
+        const double x = blocks / slots;
+        const double cost = planes / slots + (std::min(kc, top) + 2) * (0.2 + 0.15 * (std::ceil(x) - x));
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = std::min(kc, top);
+        }
+    }
+    return best;
+}
+
 template <typename R>
 StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty, int pf, int ry)
 {
@@ -49,13 +75,8 @@ StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty, int pf, int
     g.tiles_x = (nx + TX - 1) / TX;
     g.tiles_y = (ny + g.ty - 1) / g.ty;
     if (kchunk <= 0) {
-        // about two blocks per CU (256 CUs) with long z marches: measured best
-        // on 240x240x140 (fewer, longer marches amortise the two pipeline
-        // fill planes and keep halo planes in L2); chunks of >= 8 planes
         const long tiles = long(g.tiles_x) * g.tiles_y;
-        int nch = int((480 + tiles - 1) / tiles);
-        nch = std::max(1, std::min(nch, (nz + 7) / 8));
-        kchunk = (nz + nch - 1) / nch;
+        kchunk = stencil_chunk(&tiles, &nz, 1, std::is_same<R, double>::value ? kSlots64 : kSlots32);
     }
     g.kchunk = std::max(1, std::min(std::min(kchunk, nz), kMaxChunk));
     g.nchunks = (nz + g.kchunk - 1) / g.kchunk;

@@ -105,7 +105,7 @@ int stencil(helm3d_ctx* c, int variant, const OpDesc<R>& op, const cpx<R>* x, cp
     L.beta = beta;
     L.norm_part = norm_part;
     L.sink = static_cast<cpx<R>*>(c->sink);
-    TIMED(HELM3D_PROF_STENCIL, launch_stencil<R>(variant, L, c->grid, c->stream));
+    TIMED(HELM3D_PROF_STENCIL, launch_stencil<R>(variant, L, grid_of<R>(c), c->stream));
     return HELM3D_OK;
 }
 
@@ -144,8 +144,8 @@ int cycle_graph(helm3d_ctx* c, int variant, int m, const cpx<R>* V, long ld, int
     };
     const OpDesc<R>& op = op_of<R>(c);
     const void* ptrs[] = {V, c->part, c->nrm, c->gs, c->ring_dev, c->sink, skip};
-    const long ints[] = {variant, m, ld, nblk, c->N, c->grid.tiles_x, c->grid.tiles_y, c->grid.kchunk,
-                         c->grid.blocks, c->grid.ty, c->grid.pf, c->grid.ry};
+    const StencilGrid& G = grid_of<R>(c);
+    const long ints[] = {variant, m, ld, nblk, c->N, G.tiles_x, G.tiles_y, G.kchunk, G.blocks, G.ty, G.pf, G.ry};
     put(&op, sizeof(op));
     put(ptrs, sizeof(ptrs));
     put(ints, sizeof(ints));
@@ -235,7 +235,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
     // and the pinned mirror
     if (use_x0) {
         CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part));
-        TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, c->grid.blocks, 1, c->nrm, c->stream, c->small_host_dev));
+        TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, grid_of<R>(c).blocks, 1, c->nrm, c->stream, c->small_host_dev));
     } else {
         HIPCHK(launch_start<R>(b, slot(0), x, N, c->part, nblk, c->stream));
         TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, nblk, 1, c->nrm, c->stream, c->small_host_dev));
@@ -253,7 +253,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
         L.anrm = c->nrm + (j - 1);
         L.sink = static_cast<cpx<R>*>(c->sink);
         L.skip = skip;
-        TIMED(HELM3D_PROF_STENCIL, launch_stencil<R>(variant, L, c->grid, s));
+        TIMED(HELM3D_PROF_STENCIL, launch_stencil<R>(variant, L, grid_of<R>(c), s));
         // reduced dots into row (the update's coefficients) and the
         // pinned ring row, ||slot(j)||^2 into nrm[j] and the ring row
         double* hrow = device_driven ? row : c->ring_dev + size_t(j) * kGsRow;
@@ -301,7 +301,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
             if (cyc > 0) {
                 HIPCHK(launch_gmres_gate(st, c->stream));
                 CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, skip));
-                TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, c->grid.blocks, 1, c->nrm, c->stream, nullptr, skip));
+                TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, grid_of<R>(c).blocks, 1, c->nrm, c->stream, nullptr, skip));
                 HIPCHK(launch_gmres_restart(c->nrm, tol, st, c->stream));
             }
             CHK(enqueue_cycle(use_graph));
@@ -444,7 +444,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
         }
         // true residual r = b - A x into slot 0, FGMRES.m:120-124
         CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part));
-        CHK(reduce_to_small(c, c->grid.blocks, 1, 0, c->nrm));
+        CHK(reduce_to_small(c, grid_of<R>(c).blocks, 1, 0, c->nrm));
         CHK(fetch_small(c, 1));
         const double rn = std::sqrt(c->small_host[0]);
         res->relres = rn / normr0;
@@ -577,7 +577,7 @@ int bicgstab_fixed(helm3d_ctx* c, hipStream_t st, int variant, const cpx<R>* b, 
         L.y = y;
         L.alpha = R(1);
         L.sink = static_cast<cpx<R>*>(c->sink);
-        HIPCHK(launch_stencil<R>(variant, L, c->grid, st));
+        HIPCHK(launch_stencil<R>(variant, L, grid_of<R>(c), st));
         return HELM3D_OK;
     };
     HIPCHK((launch_axpby<R, R>(1.0, 0.0, b, 0.0, 0.0, r, N, false, st)));
@@ -798,7 +798,11 @@ int helm3d_set_model(helm3d_ctx* c, const int n[3], const double h[3], const int
 
     fill_opdesc(c->op64, n, c->hc, c->tab64, off, c->wn64, c->wnc, ilo, ihi);
     fill_opdesc(c->op32, n, c->hc, c->tab32, off, c->wn32, c->wnc, ilo, ihi);
-    if (!same_grid) c->grid = stencil_grid<double>(n[0], n[1], n[2], 0);
+    if (!same_grid) {
+        c->grid = stencil_grid<double>(n[0], n[1], n[2], 0);
+        c->grid32 = stencil_grid<float>(n[0], n[1], n[2], 0);
+        c->grid_auto = true;
+    }
     CHK(ensure_work(c));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->has_model = true;
@@ -814,6 +818,8 @@ int helm3d_set_launch(helm3d_ctx* c, int kchunk, int tile_rows, int prefetch, in
         return fail(HELM3D_ERR_ARG,
                     "tile_rows in {4,8}, prefetch in 1..4, kchunk >= 0, rows_per_thread 1 (or 2 with 8 rows)");
     c->grid = stencil_grid<double>(c->n[0], c->n[1], c->n[2], kchunk, tile_rows, prefetch, rows_per_thread);
+    c->grid32 = stencil_grid<float>(c->n[0], c->n[1], c->n[2], kchunk, tile_rows, prefetch, rows_per_thread);
+    c->grid_auto = false;
     CHK(ensure_work(c));
     c->inner_graph_iters = -1;
     return HELM3D_OK;
@@ -858,7 +864,7 @@ int helm3d_autotune(helm3d_ctx* c, int mode, int precision, int reps, int* kchun
     hipEvent_t e0 = nullptr, e1 = nullptr;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
-    const StencilGrid keep = c->grid;
+    const StencilGrid keep = c->grid, keep32 = c->grid32;
     StencilGrid best = keep;
     double best_t = 1e300;
     int rc = HELM3D_OK;
@@ -885,7 +891,7 @@ int helm3d_autotune(helm3d_ctx* c, int mode, int precision, int reps, int* kchun
         const int ty = sh[0], ry = sh[1];
         for (int pf : {1, 2, 3, 4}) {
             for (int kc : chunks) {
-                c->grid = stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, ry);
+                c->grid = c->grid32 = stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, ry);
                 CHK(ensure_work(c));
                 float ms = 0.f;
                 auto run = [&]() -> int {
@@ -916,6 +922,8 @@ int helm3d_autotune(helm3d_ctx* c, int mode, int precision, int reps, int* kchun
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     c->grid = rc == HELM3D_OK ? best : keep;
+    c->grid32 = rc == HELM3D_OK ? best : keep32;
+    if (rc == HELM3D_OK) c->grid_auto = false;
     CHK(ensure_work(c));
     c->inner_graph_iters = -1;  // captured graphs hold the old launch shape
     if (rc != HELM3D_OK) return rc;
