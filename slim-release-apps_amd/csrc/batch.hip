@@ -145,31 +145,8 @@ __global__ __launch_bounds__(KB) void bbicg_init_kernel(const VecItem<R>* __rest
 {
     const VecItem<R>* I = item_of(items, active);
     if (!I) return;
-    __shared__ double red[KB / 64];
-    double s2[1] = {0.0};
-    const cpx<R>* b = slot(I, bs);
-    cpx<R>* p = slot(I, ps);
-    cpx<R>* v = slot(I, vs);
-    cpx<R>* tt = slot(I, ts);
-    cpx<R>* z = slot(I, zs);
-    long lo, hi;
-    kb::range_plain(I->n, blockIdx.x, I->nblk, lo, hi);
-    const cpx<R> zero{R(0), R(0)};
-    for (long t = lo + threadIdx.x; t < hi; t += KB) {
-        const cpx<R> bv = b[t];
-        p[t] = zero;
-        v[t] = zero;
-        tt[t] = zero;
-        z[t] = zero;
-        s2[0] += double(bv.re) * double(bv.re) + double(bv.im) * double(bv.im);
-    }
-    kb::block_sum<1>(s2, red);
-    if (threadIdx.x == 0) {
-        const long G = I->nblk;
-        I->part[blockIdx.x] = s2[0];
-        I->part[G + blockIdx.x] = 0.0;
-        I->part[2 * G + blockIdx.x] = s2[0];
-    }
+    kb::bicg_init_body<R>(slot(I, bs), slot(I, ps), slot(I, vs), slot(I, ts), slot(I, zs), I->n, I->part, blockIdx.x,
+                          I->nblk);
 }
 
 template <typename R>
@@ -179,25 +156,7 @@ __global__ __launch_bounds__(KB) void bbicg_fin_kernel(const VecItem<R>* __restr
 {
     const VecItem<R>* I = item_of(items, active);
     if (!I) return;
-    const double* sc = I->sc;
-    const double ar = sc[BS_ALPHA], ai = sc[BS_ALPHA + 1];
-    const double tn = sc[BS_TT];
-    const double wr = tn > 0.0 ? sc[BS_TS] / tn : 0.0, wi = tn > 0.0 ? sc[BS_TS + 1] / tn : 0.0;
-    const cpx<R>* p = slot(I, ps);
-    const cpx<R>* r = slot(I, rs);
-    const cpx<R>* v = slot(I, vs);
-    cpx<R>* z = slot(I, zs);
-    long lo, hi;
-    kb::range_plain(I->n, blockIdx.x, I->nblk, lo, hi);
-    for (long t = lo + threadIdx.x; t < hi; t += KB) {
-        const cpx<R> pv = p[t], rv = r[t], vv = v[t], zv = z[t];
-        // s = r - alpha v
-        const double sr = double(rv.re) - (ar * double(vv.re) - ai * double(vv.im));
-        const double si = double(rv.im) - (ar * double(vv.im) + ai * double(vv.re));
-        const double zr = double(zv.re) + ar * double(pv.re) - ai * double(pv.im) + wr * sr - wi * si;
-        const double zi = double(zv.im) + ar * double(pv.im) + ai * double(pv.re) + wr * si + wi * sr;
-        z[t] = cpx<R>{R(zr), R(zi)};
-    }
+    kb::bicg_fin_body<R>(slot(I, ps), slot(I, rs), slot(I, vs), slot(I, zs), I->n, I->sc, blockIdx.x, I->nblk);
 }
 
 template <int K, typename Fn>

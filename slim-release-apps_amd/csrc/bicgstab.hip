@@ -80,6 +80,20 @@ __global__ __launch_bounds__(KB) void bicg_p_kernel(const cpx<R>* __restrict__ r
     }
 }
 
+__global__ __launch_bounds__(KB) void bicg_init_kernel(const cpx<float>* __restrict__ b, cpx<float>* __restrict__ p,
+                                                       cpx<float>* __restrict__ v, cpx<float>* __restrict__ t,
+                                                       cpx<float>* __restrict__ z, long n, double* __restrict__ part)
+{
+    kb::bicg_init_body<float>(b, p, v, t, z, n, part, blockIdx.x, gridDim.x);
+}
+
+__global__ __launch_bounds__(KB) void bicg_fin_kernel(const cpx<float>* __restrict__ p, const cpx<float>* __restrict__ r,
+                                                      const cpx<float>* __restrict__ v, cpx<float>* __restrict__ z,
+                                                      long n, const double* __restrict__ sc)
+{
+    kb::bicg_fin_body<float>(p, r, v, z, n, sc, blockIdx.x, gridDim.x);
+}
+
 }  // namespace
 
 template <typename R>
@@ -114,6 +128,20 @@ hipError_t launch_bicg_p(const cpx<R>* r, const cpx<R>* v, cpx<R>* p, long n, co
                          int rho_old, hipStream_t st)
 {
     hipLaunchKernelGGL((bicg_p_kernel<R>), dim3(krylov_blocks(n)), dim3(KB), 0, st, r, v, p, n, sc, rho_new, rho_old);
+    return hipGetLastError();
+}
+
+hipError_t launch_bicg_init(const cpx<float>* b, cpx<float>* p, cpx<float>* v, cpx<float>* t, cpx<float>* z, long n,
+                            double* part, int nblk, hipStream_t st)
+{
+    hipLaunchKernelGGL(bicg_init_kernel, dim3(nblk), dim3(KB), 0, st, b, p, v, t, z, n, part);
+    return hipGetLastError();
+}
+
+hipError_t launch_bicg_fin(const cpx<float>* p, const cpx<float>* r, const cpx<float>* v, cpx<float>* z, long n,
+                           const double* sc, int nblk, hipStream_t st)
+{
+    hipLaunchKernelGGL(bicg_fin_kernel, dim3(nblk), dim3(KB), 0, st, p, r, v, z, n, sc);
     return hipGetLastError();
 }
 

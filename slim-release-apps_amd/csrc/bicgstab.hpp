@@ -13,8 +13,8 @@ constexpr int BS_RHO1 = 3;   // second triple
 constexpr int BS_RV = 6;     // (rhat, v)
 constexpr int BS_TS = 8;     // (t, s) re, im ; BS_TS + 2: ||t||^2
 constexpr int BS_TT = 10;
-constexpr int BS_RS = 11;    // (rhat, s) re, im (fused batched form)
-constexpr int BS_RT = 13;    // (rhat, t) re, im (fused batched form)
+constexpr int BS_RS = 11;    // (rhat, s) re, im (fused form)
+constexpr int BS_RT = 13;    // (rhat, t) re, im (fused form)
 constexpr int BS_ALPHA = 15;
 constexpr int BS_OMEGA = 17;
 constexpr int BS_SLOTS = 20;
@@ -38,5 +38,12 @@ hipError_t launch_bicg_xr(const cpx<R>* p, const cpx<R>* s, const cpx<R>* t, con
 template <typename R>
 hipError_t launch_bicg_p(const cpx<R>* r, const cpx<R>* v, cpx<R>* p, long n, const double* sc, int rho_new,
                          int rho_old, hipStream_t st);
+
+// Start and last z update of the fused iteration (epilogues 3 and 4 of the
+// stencil); see the bodies in kbody.hpp.
+hipError_t launch_bicg_init(const cpx<float>* b, cpx<float>* p, cpx<float>* v, cpx<float>* t, cpx<float>* z, long n,
+                            double* part, int nblk, hipStream_t st);
+hipError_t launch_bicg_fin(const cpx<float>* p, const cpx<float>* r, const cpx<float>* v, cpx<float>* z, long n,
+                           const double* sc, int nblk, hipStream_t st);
 
 }  // namespace helm3d

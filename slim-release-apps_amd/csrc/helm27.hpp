@@ -82,6 +82,9 @@ StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 4, int pf 
 template <typename R>
 hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g, hipStream_t s);
 
+// The fused BiCGStab forms (epi 3 or 4, no DERIV) for one vector.
+hipError_t launch_stencil_fused(int variant, int epi, StencilLaunch<float> L, const StencilGrid& g, hipStream_t s);
+
 // One launch over nitems device-resident StencilLaunch items (operators
 // without DERIV); item it owns blocks [first[it], first[it+1]) of `blocks`,
 // launched with its own tiles_x/tiles_y/kchunk and the common shape (ty, pf,

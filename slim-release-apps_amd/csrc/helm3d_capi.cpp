@@ -550,59 +550,67 @@ int bicgstab_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* z, doub
     return HELM3D_OK;
 }
 
-// Fixed-length BiCGStab (exactly `iters` iterations, no host reads, no
-// profiling events) on stream st: the body captured into a HIP graph.  The
-// breakdown guards of the scalar kernels (zero denominators give zero steps)
-// make a zero right-hand side return z = 0.
-template <typename R>
-int bicgstab_fixed(helm3d_ctx* c, hipStream_t st, int variant, const cpx<R>* b, cpx<R>* z, long iters)
+// Fixed-length complex64 BiCGStab (exactly `iters` iterations, no host reads,
+// no profiling events) on stream st: the body captured into a HIP graph.  An
+// iteration is two stencil launches with every vector update fused in
+// (epilogues 3 and 4) and their reductions, 120 B a point; with separate dot
+// and update passes it was nine launches and 184 B.  b serves as rhat and as
+// the first residual.  The guards of the scalar forms (zero denominators give
+// zero steps) make a zero right-hand side return z = 0.
+int bicgstab_fixed(helm3d_ctx* c, hipStream_t st, int variant, const cpx<float>* b, cpx<float>* z, long iters)
 {
     const long N = c->N;
     const long ld = slot_ld(N);
-    cpx<R>* W = bicg_of<R>(c).p;
-    cpx<R>* r = W;
-    cpx<R>* rh = W + ld;
-    cpx<R>* p = W + 2 * ld;
-    cpx<R>* v = W + 3 * ld;
-    cpx<R>* sv = W + 4 * ld;
-    cpx<R>* t = W + 5 * ld;
-    const OpDesc<R>& op = op_of<R>(c);
+    cpx<float>* W = c->BC32.p;
+    cpx<float>* r[2] = {W, W + ld};
+    cpx<float>* p[2] = {W + 2 * ld, W + 3 * ld};
+    cpx<float>* v[2] = {W + 4 * ld, W + 5 * ld};
+    cpx<float>* t = W + 6 * ld;
+    const StencilGrid& G = c->grid32;
     const int nblk = krylov_blocks(N);
     double* sc = c->bsc;
-    const cpx<R>* none = nullptr;
-    auto sten = [&](const cpx<R>* x, cpx<R>* y) -> int {
-        StencilLaunch<R> L{};
-        L.op = op;
-        L.x = x;
-        L.y = y;
-        L.alpha = R(1);
-        L.sink = static_cast<cpx<R>*>(c->sink);
-        HIPCHK(launch_stencil<R>(variant, L, grid_of<R>(c), st));
-        return HELM3D_OK;
-    };
-    HIPCHK((launch_axpby<R, R>(1.0, 0.0, b, 0.0, 0.0, r, N, false, st)));
-    HIPCHK((launch_axpby<R, R>(1.0, 0.0, b, 0.0, 0.0, rh, N, false, st)));
-    HIPCHK((launch_axpby<R, R>(1.0, 0.0, b, 0.0, 0.0, p, N, false, st)));
-    HIPCHK((launch_axpby<R, R>(0.0, 0.0, none, 0.0, 0.0, z, N, false, st)));
-    PairArgs<R> P0{{rh, nullptr}, {r, nullptr}};
-    HIPCHK(launch_dots_pairs<R>(P0, 1, true, N, c->part, nblk, st));
+    HIPCHK(launch_bicg_init(b, p[0], v[0], t, z, N, c->part, nblk, st));
     HIPCHK(launch_reduce(c->part, nblk, 3, sc + BS_RHO0, st));
     for (long it = 0; it < iters; ++it) {
-        const int cur = (it & 1) ? BS_RHO1 : BS_RHO0;
-        const int nxt = (it & 1) ? BS_RHO0 : BS_RHO1;
-        CHK(sten(p, v));
-        PairArgs<R> P1{{rh, nullptr}, {v, nullptr}};
-        HIPCHK(launch_dots_pairs<R>(P1, 1, false, N, c->part, nblk, st));
-        HIPCHK(launch_reduce(c->part, nblk, 2, sc + BS_RV, st));
-        HIPCHK(launch_bicg_s<R>(r, v, sv, N, sc, cur, st));
-        CHK(sten(sv, t));
-        PairArgs<R> P2{{t, nullptr}, {sv, nullptr}};
-        HIPCHK(launch_dots_pairs<R>(P2, 1, true, N, c->part, nblk, st));
-        HIPCHK(launch_reduce(c->part, nblk, 3, sc + BS_TS, st));
-        HIPCHK(launch_bicg_xr<R>(p, sv, t, rh, z, r, N, sc, c->part, nblk, st));
-        HIPCHK(launch_reduce(c->part, nblk, 3, sc + nxt, st));
-        if (it + 1 < iters) HIPCHK(launch_bicg_p<R>(r, v, p, N, sc, nxt, cur, st));
+        // iteration it reads r, p, v of the one before from the cur slots and
+        // writes the nxt slots (the stencil reads them at halo points)
+        const int cur = int(it & 1), nxt = cur ^ 1;
+        StencilLaunch<float> A{};
+        A.op = c->op32;
+        A.alpha = 1.0f;
+        A.f0 = it == 0 ? b : r[cur];
+        A.f1 = p[cur];
+        A.f2 = v[cur];
+        A.f3 = t;
+        A.o2 = p[nxt];
+        A.o3 = r[nxt];
+        A.zz = z;
+        A.y = v[nxt];
+        A.rh = b;
+        A.sc = sc;
+        A.rho_new = cur == 0 ? BS_RHO0 : BS_RHO1;
+        A.rho_old = cur == 0 ? BS_RHO1 : BS_RHO0;
+        A.first = it == 0;
+        A.norm_part = c->part;
+        A.sink = static_cast<cpx<float>*>(c->sink);
+        HIPCHK(launch_stencil_fused(variant, 3, A, G, st));
+        HIPCHK(launch_reduce(c->part, G.blocks, 2, sc + BS_RV, st));
+        StencilLaunch<float> B{};
+        B.op = c->op32;
+        B.alpha = 1.0f;
+        B.f0 = r[nxt];
+        B.f1 = v[nxt];
+        B.y = t;
+        B.rh = b;
+        B.sc = sc;
+        B.rho_new = A.rho_new;
+        B.norm_part = c->part;
+        B.sink = A.sink;
+        HIPCHK(launch_stencil_fused(variant, 4, B, G, st));
+        HIPCHK(launch_reduce(c->part, G.blocks, 7, sc + BS_TS, st));
     }
+    const int last = int(iters & 1);  // slots of the last iteration's p, r, v
+    if (iters > 0) HIPCHK(launch_bicg_fin(p[last], r[last], v[last], z, N, sc, nblk, st));
     return HELM3D_OK;
 }
 
@@ -611,9 +619,9 @@ int bicgstab_fixed(helm3d_ctx* c, hipStream_t st, int variant, const cpx<R>* b, 
 // this variant and length).
 int inner_fixed_c64(helm3d_ctx* c, int variant, long iters)
 {
-    CHK(ensure_vecs(c->BC32, c->N, 6));
+    CHK(ensure_vecs(c->BC32, c->N, 7));
     CHK(ensure_t(&c->bsc, &c->bsc_cap, BS_SLOTS));
-    if (!c->use_graphs) return bicgstab_fixed<float>(c, c->stream, variant, c->T32a.p, c->T32b.p, iters);
+    if (!c->use_graphs) return bicgstab_fixed(c, c->stream, variant, c->T32a.p, c->T32b.p, iters);
     if (!c->inner_graph || c->inner_graph_variant != variant || c->inner_graph_iters != iters) {
         if (c->inner_graph) {
             HIPCHK(hipGraphExecDestroy(c->inner_graph));
@@ -622,7 +630,7 @@ int inner_fixed_c64(helm3d_ctx* c, int variant, long iters)
         if (!c->cap_stream) HIPCHK(hipStreamCreateWithFlags(&c->cap_stream, hipStreamNonBlocking));
         hipGraph_t g = nullptr;
         HIPCHK(hipStreamBeginCapture(c->cap_stream, hipStreamCaptureModeThreadLocal));
-        const int st = bicgstab_fixed<float>(c, c->cap_stream, variant, c->T32a.p, c->T32b.p, iters);
+        const int st = bicgstab_fixed(c, c->cap_stream, variant, c->T32a.p, c->T32b.p, iters);
         const hipError_t e = hipStreamEndCapture(c->cap_stream, &g);
         if (st != HELM3D_OK) {
             if (g) (void)hipGraphDestroy(g);

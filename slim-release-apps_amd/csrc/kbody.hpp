@@ -323,5 +323,56 @@ __device__ __forceinline__ void bicg_xr_body(const cpx<R>* __restrict__ p, const
     }
 }
 
+// Start of a fused BiCGStab solve from z = 0 with r = rhat = b: p = v = t = z
+// = 0 and the partials of ||b||^2 in columns 0 and 2 (column 1 zero).
+template <typename R>
+__device__ __forceinline__ void bicg_init_body(const cpx<R>* __restrict__ b, cpx<R>* __restrict__ p,
+                                               cpx<R>* __restrict__ v, cpx<R>* __restrict__ tt,
+                                               cpx<R>* __restrict__ z, long n, double* __restrict__ part, int blk,
+                                               int G)
+{
+    __shared__ double red[KB / 64];
+    double s2[1] = {0.0};
+    long lo, hi;
+    range_plain(n, blk, G, lo, hi);
+    const cpx<R> zero{R(0), R(0)};
+    for (long t = lo + threadIdx.x; t < hi; t += KB) {
+        const cpx<R> bv = b[t];
+        p[t] = zero;
+        v[t] = zero;
+        tt[t] = zero;
+        z[t] = zero;
+        s2[0] += double(bv.re) * double(bv.re) + double(bv.im) * double(bv.im);
+    }
+    block_sum<1>(s2, red);
+    if (threadIdx.x == 0) {
+        part[blk] = s2[0];
+        part[long(G) + blk] = 0.0;
+        part[2 * long(G) + blk] = s2[0];
+    }
+}
+
+// Last z update of the fused iteration: z += alpha p + omega (r - alpha v).
+template <typename R>
+__device__ __forceinline__ void bicg_fin_body(const cpx<R>* __restrict__ p, const cpx<R>* __restrict__ r,
+                                              const cpx<R>* __restrict__ v, cpx<R>* __restrict__ z, long n,
+                                              const double* __restrict__ sc, int blk, int G)
+{
+    const double ar = sc[BS_ALPHA], ai = sc[BS_ALPHA + 1];
+    const double tn = sc[BS_TT];
+    const double wr = tn > 0.0 ? sc[BS_TS] / tn : 0.0, wi = tn > 0.0 ? sc[BS_TS + 1] / tn : 0.0;
+    long lo, hi;
+    range_plain(n, blk, G, lo, hi);
+    for (long t = lo + threadIdx.x; t < hi; t += KB) {
+        const cpx<R> pv = p[t], rv = r[t], vv = v[t], zv = z[t];
+        // s = r - alpha v
+        const double sr = double(rv.re) - (ar * double(vv.re) - ai * double(vv.im));
+        const double si = double(rv.im) - (ar * double(vv.im) + ai * double(vv.re));
+        const double zr = double(zv.re) + ar * double(pv.re) - ai * double(pv.im) + wr * sr - wi * si;
+        const double zi = double(zv.im) + ar * double(pv.im) + ai * double(pv.re) + wr * si + wi * sr;
+        z[t] = cpx<R>{R(zr), R(zi)};
+    }
+}
+
 }  // namespace kb
 }  // namespace helm3d
