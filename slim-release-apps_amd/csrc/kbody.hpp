@@ -44,6 +44,107 @@ __device__ inline void block_sum(double (&v)[NV], double* red /* [KB/64][NV] */)
     }
 }
 
+// Sums of NV values per lane over a wave, one or two lanes ending up with each:
+// at every step a lane hands half of its values to its partner and keeps the
+// other half, so NV + NV/2 + ... values cross lanes instead of 6 NV.  The
+// exchange over 32 and 16 lanes is the swap of two registers; below 16 lanes
+// the partner is lane ^ 8, ^ 7, ^ 2, ^ 1 (row rotate, half mirror, quad
+// permutes).  Returns the value of this lane and its index q (q < 0: none).
+__device__ inline double dpp_mov(double v, int sel)
+{
+    const long long b = __double_as_longlong(v);
+    int lo, hi;
+    switch (sel) {
+    case 8:
+        lo = __builtin_amdgcn_mov_dpp(int(b), 0x128, 0xf, 0xf, true);
+        hi = __builtin_amdgcn_mov_dpp(int(b >> 32), 0x128, 0xf, 0xf, true);
+        break;
+    case 4:
+        lo = __builtin_amdgcn_mov_dpp(int(b), 0x141, 0xf, 0xf, true);
+        hi = __builtin_amdgcn_mov_dpp(int(b >> 32), 0x141, 0xf, 0xf, true);
+        break;
+    case 2:
+        lo = __builtin_amdgcn_mov_dpp(int(b), 0x4E, 0xf, 0xf, true);
+        hi = __builtin_amdgcn_mov_dpp(int(b >> 32), 0x4E, 0xf, 0xf, true);
+        break;
+    default:
+        lo = __builtin_amdgcn_mov_dpp(int(b), 0xB1, 0xf, 0xf, true);
+        hi = __builtin_amdgcn_mov_dpp(int(b >> 32), 0xB1, 0xf, 0xf, true);
+        break;
+    }
+    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// a of the lanes whose bit M is clear and of their partners, added, in those
+// lanes; b likewise in the others.
+template <int M>
+__device__ inline double half_step(double a, double b, int lane)
+{
+    if constexpr (M >= 16) {
+        const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+        auto swap = [](unsigned p, unsigned q) {
+            if constexpr (M == 32) return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+            else return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+        };
+        const auto lo = swap(unsigned(x), unsigned(y));
+        const auto hi = swap(unsigned(x >> 32), unsigned(y >> 32));
+        const double p = __longlong_as_double((static_cast<long long>(hi[0]) << 32) | lo[0]);
+        const double q = __longlong_as_double((static_cast<long long>(hi[1]) << 32) | lo[1]);
+        return p + q;
+    } else {
+        const bool up = lane & M;
+        const double keep = up ? b : a, send = up ? a : b;
+        return keep + dpp_mov(send, M);
+    }
+}
+
+template <int M, int CNT>
+__device__ inline double wave_sums_step(double (&v)[CNT], int lane, int& base, int& end)
+{
+    if constexpr (M == 0) {
+        return v[0];
+    } else {
+        constexpr int H = (CNT + 1) / 2;
+        double w[H];
+#pragma unroll
+        for (int i = 0; i < H; ++i) w[i] = half_step<M>(v[i], CNT == 1 ? v[i] : (i + H < CNT ? v[i + H] : 0.0), lane);
+        if (CNT > 1) {
+            if (lane & M) base += H;
+            else end = min(end, base + H);
+        }
+        return wave_sums_step<M / 2, H>(w, lane, base, end);
+    }
+}
+
+template <int NV>
+__device__ inline double wave_sums(double (&v)[NV], int lane, int& q)
+{
+    static_assert(NV <= 64, "one value per lane");
+    int base = 0, end = NV;
+    const double s = wave_sums_step<32, NV>(v, lane, base, end);
+    q = base < end ? base : -1;
+    return s;
+}
+
+// Block-wide sums of NV values per thread into part[q * G + b], q < NV: waves
+// by wave_sums, then one thread per value adds the waves in order.
+template <int NV>
+__device__ inline void block_sum_store(double (&v)[NV], double* red /* [KB/64][NV] */, double* __restrict__ part,
+                                       int b, int G)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    int q;
+    const double s = wave_sums<NV>(v, lane, q);
+    if (q >= 0) red[wid * NV + q] = s;
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double t = red[threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < KB / 64; ++w) t += red[w * NV + threadIdx.x];
+        part[long(threadIdx.x) * G + b] = t;
+    }
+}
+
 // Contiguous range [lo, hi) of block b (even length).
 __device__ inline void range_even(long n, int b, int G, long& lo, long& hi)
 {
@@ -117,11 +218,7 @@ __device__ __forceinline__ void dots_body(const cpx<R>* __restrict__ V, long ldv
 #pragma unroll
         for (int c = 0; c < K; ++c) acc_dot(acc[2 * c], acc[2 * c + 1], ld_basis<NT>(&V[c * ldv + t]), w0);
     }
-    block_sum<2 * K>(acc, red);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int q = 0; q < 2 * K; ++q) part[long(q) * G + b] = acc[q];
-    }
+    block_sum_store<2 * K>(acc, red, part, b, G);
 }
 
 // w <- w - sum_{c<K} a_c v_c; partial ||w||^2 in column 0.

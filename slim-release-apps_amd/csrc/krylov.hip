@@ -375,8 +375,10 @@ int dots_blocks(long n)
 {
     const long kb = krylov_blocks(n);
     if (kb <= kInBlockDots) return int(kb);
-    const long b = std::max((n + KB * 32 - 1) / (KB * 32), std::min(kb, 512L));
-    return int(std::min(b, long(kMaxPartials)));
+    long per = 4;
+    auto blocks = [&]() { return (n + KB * per - 1) / (KB * per); };
+    while (per < 16 && blocks() > 1100) per *= 2;
+    return int(std::min(blocks(), long(kMaxPartials)));
 }
 
 int update_blocks(long n)

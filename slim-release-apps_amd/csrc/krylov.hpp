@@ -17,11 +17,13 @@ int krylov_blocks(long n);
 
 // Blocks of the Gram-Schmidt passes over complex128 vectors long enough for
 // the separate dots reduction (krylov_blocks(n) > kInBlockDots; shorter ones
-// get krylov_blocks(n)).  The dots pass reduces 2K partial sums per block and
-// streams fastest with about 32 points per thread (at least min(krylov_blocks,
-// 512) blocks, at most kMaxPartials); the update pass, one partial per block,
-// with about 2 (at most kMaxUpdateBlocks).  Measured on 8,064,000 points:
-// dots 6.0 -> 6.4 TB/s at K = 20, update 5.2 -> 5.4 TB/s.
+// get krylov_blocks(n)).  The dots pass ends each block with sums of 2K values
+// over its waves and streams fastest with 500 to 1100 blocks of 4, 8 or 16
+// points per thread (16 on longer vectors, at most kMaxPartials blocks); the
+// update pass, one partial per block, with about 2 points per thread (at most
+// kMaxUpdateBlocks).  K = 20 cycles, dots average per pass: 84^3 points 4 / 16
+// / 32 points per thread 20.7 / 22.0 / 33.1 us, 150 x 150 x 100 4 / 8 / 16
+// 72.4 / 69.7 / 79.0, 240 x 240 x 140 8 / 16 / 32 263 / 237 / 254.
 constexpr int kMaxUpdateBlocks = 16384;
 static_assert(kMaxUpdateBlocks <= kMaxPartials * 2 * kMaxBasis, "update partials fit the dots partials buffer");
 int dots_blocks(long n);
