@@ -48,6 +48,34 @@ struct StencilLaunch {
     const int* skip;  // optional (device): the launch does nothing while *skip != 0
 };
 
+struct GmresDevState;
+
+// Arnoldi step of the device-driven GMRES on small grids (EPI 5): y = H x /
+// ||x||, then the dots of y with the basis slots, in one launch.
+//   npart, npn  partial sums of ||x||^2, added by every wave in one order
+//   nrm, row    ||x||^2 stored by block 0 for the update pass and the least
+//               squares (row optional)
+//   start       0: an inner step; 1: first step of a solve, 2: of a restarted
+//               cycle: block 0 opens the state st, and the launch does nothing
+//               on a zero residual (1) or one below tol (2)
+//   V, ldv, k   basis slots 0 .. k-1 (k <= kStepMaxK)
+//   dpart       partials of the 2k sums: dpart[q * blocks + block]
+constexpr int kStepMaxK = 8;
+template <typename R>
+struct StepArgs {
+    const double* npart;
+    int npn;
+    int start;
+    double* nrm;
+    double* row;
+    GmresDevState* st;
+    double tol;
+    const cpx<R>* V;
+    long ldv;
+    int k;
+    double* dpart;
+};
+
 // Launch shape: 64 x ty column tiles, z chunks of kchunk planes, pf planes of
 // loads in flight, ry rows per thread (2 only with ty = 8: 256 threads per
 // tile instead of 512).
@@ -81,6 +109,11 @@ StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 4, int pf 
 
 template <typename R>
 hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g, hipStream_t s);
+
+// The Arnoldi step form (EPI 5, no DERIV).
+template <typename R>
+hipError_t launch_stencil_step(int variant, StencilLaunch<R> L, const StepArgs<R>& X, const StencilGrid& g,
+                               hipStream_t s);
 
 // The fused BiCGStab forms (epi 3 or 4, no DERIV) for one vector.
 hipError_t launch_stencil_fused(int variant, int epi, StencilLaunch<float> L, const StencilGrid& g, hipStream_t s);

@@ -30,8 +30,9 @@
 
 #include <type_traits>
 
-#include "bicgstab.hpp"
 #include "helm27.hpp"
+#include "kbody.hpp"
+#include "krylov.hpp"
 
 namespace helm3d {
 
@@ -98,9 +99,12 @@ __device__ inline Cd cd_div(Cd a, Cd b)
 //      EPI 4 launch
 //   4: x = s = r - alpha v formed while staging, y = t = H s, partials
 //      (t, s), ||t||^2, (rhat, s) and (rhat, t)
+// 5 is an Arnoldi step (StepArgs X): EPI 0 with the scale summed from partials
+// and, after the march, the dots of the block's outputs with the basis.
 // The body runs one block `lin` of a launch of `G` blocks described by L.
 template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY = 1>
-__device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int lin, const int G)
+__device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int lin, const int G,
+                                            const StepArgs<R>* X = nullptr)
 {
     static_assert(RY == 1 || RY == 2, "one or two rows per thread");
     static_assert(TY % RY == 0, "rows per thread divide the tile rows");
@@ -284,7 +288,32 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
 #pragma unroll
     for (int r = 0; r < RY; ++r) Xlast[r] = Rlast[r] = Dlast[r] = zero<R>();
     // output scale: alpha, or alpha / sqrt(*anrm) with the norm held on the device
-    const R alpha = (EPI <= 1 && L.anrm) ? R(double(L.alpha) / sqrt(*L.anrm)) : L.alpha;
+    R alpha = (EPI <= 1 && L.anrm) ? R(double(L.alpha) / sqrt(*L.anrm)) : L.alpha;
+    if constexpr (EPI == 5) {
+        // every wave adds the partials of ||x||^2 in the same order
+        double s = 0.0;
+        for (int q = tx; q < X->npn; q += 64) s += X->npart[q];
+        s = kb::wave_sum(s);
+        bool stop = false;
+        if (X->start) {
+            const double b = sqrt(s);
+            stop = X->start == 1 ? b == 0.0 : b / X->st->normr0 < X->tol;
+            if (lin == 0 && tid == 0) {
+                if (X->start == 1) {
+                    X->st->normr0 = b;
+                    X->st->hlast = 1.0;
+                }
+                X->st->beta = b;
+                X->st->skip = stop ? 1 : 0;
+            }
+        }
+        if (lin == 0 && tid == 0) {
+            *X->nrm = s;
+            if (X->row) *X->row = s;
+        }
+        if (stop) return;  // the same decision in every block
+        alpha = R(double(L.alpha) / sqrt(s));
+    }
 
     // One register set: halo slots of plane q and the own-point operands of
     // plane q-1 (the plane output when q is staged).  Every load is issued
@@ -644,6 +673,39 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
         const int q = k0 - 1 + trp * PF;
 #pragma unroll
         for (int p = 0; p < PF; ++p) step(q + p, trp * PF + p, S[p]);
+    }
+
+    if constexpr (EPI == 5) {
+        // dots of the block's outputs (each thread its own, from cache) with
+        // the basis slots; a slot's loads of a point are issued together
+        double da[2 * kStepMaxK];
+#pragma unroll
+        for (int q = 0; q < 2 * kStepMaxK; ++q) da[q] = 0.0;
+        const int nk = X->k;
+        for (int kk = k0; kk < k1; ++kk) {
+#pragma unroll
+            for (int r = 0; r < RY; ++r) {
+                if (!active[r]) continue;
+                const long t = long(kk) * plane + offc[r];
+                const cpx<R> w = L.y[t];
+                cpx<R> v[kStepMaxK];
+#pragma unroll
+                for (int c = 0; c < kStepMaxK; ++c) v[c] = c < nk ? X->V[c * X->ldv + t] : zero<R>();
+#pragma unroll
+                for (int c = 0; c < kStepMaxK; ++c)
+                    if (c < nk) kb::acc_dot(da[2 * c], da[2 * c + 1], v[c], w);
+            }
+        }
+        __shared__ double dred[NT / 64][2 * kStepMaxK];
+        int q;
+        const double s = kb::wave_sums<2 * kStepMaxK>(da, tx, q);
+        if (q >= 0) dred[tw][q] = s;
+        __syncthreads();
+        if (tid < 2 * nk) {
+            double t = dred[0][tid];
+            for (int w = 1; w < NT / 64; ++w) t += dred[w][tid];
+            X->dpart[long(tid) * G + lin] = t;
+        }
     }
 
     // optional per-block partials (deterministic two-stage reduction):

@@ -1,0 +1,58 @@
+// Arnoldi steps of the device-driven GMRES on small grids: matvec and dots in
+// one launch (EPI 5 of the stencil body).  On a coarse multigrid level a launch
+// takes a few microseconds whatever it does, so the step is two launches (this
+// and the update pass) instead of four: the norm of the input is summed from
+// the update pass's partials here, the dots from this launch's partials there.
+#include "helm27_body.hpp"
+
+namespace helm3d {
+
+namespace {
+
+template <typename R, bool ADJ, bool WNC, int TY, int PF, int RY>
+__global__ __launch_bounds__(TX* TY / RY) void helm27_step_kernel(StencilLaunch<R> L, StepArgs<R> X)
+{
+    helm27_body<R, ADJ, false, WNC, TY, PF, 5, RY>(L, blockIdx.x, gridDim.x, &X);
+}
+
+// one or two planes in flight: the small grids march a few planes per block
+template <typename R, bool A, bool W>
+hipError_t launch_shape(const StencilLaunch<R>& L, const StepArgs<R>& X, const StencilGrid& g, hipStream_t s)
+{
+    const dim3 grid(g.blocks);
+    const bool two = g.pf >= 2;
+    if (g.ty == 8 && g.ry == 2) {
+        if (two) hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 2, 2>), grid, dim3(TX * 4), 0, s, L, X);
+        else hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 1, 2>), grid, dim3(TX * 4), 0, s, L, X);
+    } else if (g.ty == 8) {
+        if (two) hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 2, 1>), grid, dim3(TX * 8), 0, s, L, X);
+        else hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 1, 1>), grid, dim3(TX * 8), 0, s, L, X);
+    } else {
+        if (two) hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 4, 2, 1>), grid, dim3(TX * 4), 0, s, L, X);
+        else hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 4, 1, 1>), grid, dim3(TX * 4), 0, s, L, X);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+template <typename R>
+hipError_t launch_stencil_step(int variant, StencilLaunch<R> L, const StepArgs<R>& X, const StencilGrid& g,
+                               hipStream_t s)
+{
+    L.tiles_x = g.tiles_x;
+    L.tiles_y = g.tiles_y;
+    L.kchunk = g.kchunk;
+    if ((variant & VAR_DERIV) || X.k < 1 || X.k > kStepMaxK) return hipErrorInvalidValue;
+    const bool adj = variant & VAR_ADJ, wnc = variant & VAR_WNC;
+    if (!adj && !wnc) return launch_shape<R, false, false>(L, X, g, s);
+    if (!adj) return launch_shape<R, false, true>(L, X, g, s);
+    return wnc ? launch_shape<R, true, true>(L, X, g, s) : launch_shape<R, true, false>(L, X, g, s);
+}
+
+template hipError_t launch_stencil_step<double>(int, StencilLaunch<double>, const StepArgs<double>&,
+                                                const StencilGrid&, hipStream_t);
+template hipError_t launch_stencil_step<float>(int, StencilLaunch<float>, const StepArgs<float>&,
+                                               const StencilGrid&, hipStream_t);
+
+}  // namespace helm3d

@@ -134,9 +134,9 @@ namespace helm3d {
 // shape, cycle length and every buffer address the steps use.
 template <typename R, typename Rec>
 int cycle_graph(helm3d_ctx* c, int variant, int m, const cpx<R>* V, long ld, int nblk, const int* skip,
-                Rec&& record)
+                Rec&& record, int which = 0, double tol = 0.0)
 {
-    const int p = std::is_same<R, double>::value ? 0 : 1;
+    const int p = (std::is_same<R, double>::value ? 0 : 1) + 2 * which;
     std::vector<unsigned char> key;
     auto put = [&](const void* a, size_t n) {
         const auto* b = static_cast<const unsigned char*>(a);
@@ -149,6 +149,7 @@ int cycle_graph(helm3d_ctx* c, int variant, int m, const cpx<R>* V, long ld, int
     put(&op, sizeof(op));
     put(ptrs, sizeof(ptrs));
     put(ints, sizeof(ints));
+    put(&tol, sizeof(tol));
     if (!c->cyc_graph[p] || c->cyc_key[p] != key) {
         if (c->cyc_graph[p]) {
             HIPCHK(hipGraphExecDestroy(c->cyc_graph[p]));
@@ -231,6 +232,64 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
     GmresDevState* st = c->gst;
     const int* skip = device_driven ? &st->skip : nullptr;
 
+    // Device-driven solves of short vectors: two launches per Arnoldi step.
+    // The step launch (matvec and dots) sums the partials that the update pass
+    // (or the start) left of its input's norm, the update pass the dots; the
+    // first step of a cycle takes the stop decisions, the least squares the
+    // norm of the last slot.  Partials: norms at the front, dots behind them.
+    const StencilGrid& G = grid_of<R>(c);
+    if (device_driven && nblk <= kInBlockDots && G.blocks <= kStepBlocks && m <= kStepMaxK) {
+        double* dpart = c->part + kStepBlocks;
+        auto steps = [&](hipStream_t s, int start, int npn) -> int {
+            for (int j = 1; j <= m; ++j) {
+                StencilLaunch<R> L{};
+                L.op = op;
+                L.x = slot(j - 1);
+                L.y = slot(j);
+                L.alpha = R(1);
+                L.sink = static_cast<cpx<R>*>(c->sink);
+                L.skip = start == 1 && j == 1 ? nullptr : &st->skip;
+                StepArgs<R> X{};
+                X.npart = c->part;
+                X.npn = j == 1 ? npn : nblk;
+                X.start = j == 1 ? start : 0;
+                X.nrm = c->nrm + (j - 1);
+                X.row = j == 1 ? nullptr : c->gs + size_t(j - 1) * kGsRow + 2 * (j - 1);
+                X.st = st;
+                X.tol = tol;
+                X.V = V;
+                X.ldv = ld;
+                X.k = j;
+                X.dpart = dpart;
+                TIMED(HELM3D_PROF_STENCIL, launch_stencil_step<R>(variant, L, X, G, s));
+                TIMED(HELM3D_PROF_UPDATE,
+                      launch_update<R>(V, ld, j, nullptr, CoefPack{}, slot(j), N, c->part, nblk, s, c->nrm, dpart,
+                                       G.blocks, c->gs + size_t(j) * kGsRow, &st->skip));
+            }
+            HIPCHK(launch_gmres_lsq(c->gs, kGsRow, m, tol, st, s, c->part, nblk));
+            return HELM3D_OK;
+        };
+        for (long cyc = 0; (1 + cyc * long(m)) / m < maxit; ++cyc) {
+            const bool resid = cyc > 0 || use_x0;
+            if (resid) CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, cyc > 0 ? skip : nullptr));
+            else HIPCHK(launch_start<R>(b, slot(0), x, N, c->part, nblk, c->stream));
+            const int start = cyc > 0 ? 2 : 1, npn = resid ? G.blocks : nblk;
+            if (c->use_graphs && !c->prof)
+                CHK(cycle_graph<R>(c, variant, m, V, ld, npn, skip,
+                                   [&](hipStream_t s) { return steps(s, start, npn); },
+                                   cyc > 0 ? 3 : (resid ? 2 : 1), tol));
+            else
+                CHK(steps(c->stream, start, npn));
+            TIMED(HELM3D_PROF_COMBINE,
+                  launch_combine_dev<R>(V, ld, m, st->coef, &st->kept, x, N, nblk_u, c->stream, nullptr));
+        }
+        res->iters = -1;
+        res->cycles = -1;
+        res->relres = res->quasi = std::nan("");
+        res->converged = false;
+        return HELM3D_OK;
+    }
+
     // r0 = b - A x0, or b with x = 0 (FGMRES.m:57-62); ||r0||^2 into nrm[0]
     // and the pinned mirror
     if (use_x0) {
@@ -262,12 +321,12 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
             // pass (partials one column up, clear of the norm partials)
             TIMED(HELM3D_PROF_DOTS, launch_dots<R>(V, ld, j, slot(j), N, c->part + nblk, nblk, s, skip));
             TIMED(HELM3D_PROF_UPDATE, launch_update<R>(V, ld, j, nullptr, CoefPack{}, slot(j), N, c->part,
-                                                       nblk, s, c->nrm, c->part + nblk, hrow, skip));
+                                                       nblk, s, c->nrm, c->part + nblk, nblk, hrow, skip));
         } else {
             TIMED(HELM3D_PROF_DOTS, launch_dots<R>(V, ld, j, slot(j), N, c->part, nblk_d, s, skip));
             TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, nblk_d, 2 * j, row, s, hrow, skip));
             TIMED(HELM3D_PROF_UPDATE, launch_update<R>(V, ld, j, row, CoefPack{}, slot(j), N, c->part, nblk_u, s,
-                                                       c->nrm, nullptr, nullptr, skip));
+                                                       c->nrm, nullptr, 0, nullptr, skip));
         }
         const int nu = nblk <= kInBlockDots ? nblk : nblk_u;
         TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, nu, 1, c->nrm + j, s, hrow + 2 * j, skip));

@@ -101,6 +101,7 @@ __global__ __launch_bounds__(KB) void combine_dev_kernel(const cpx<R>* __restric
 {
     if (skip && *skip) return;
     const int kk = min(*kept, K);
+    if (kk == 0) return;
     double pr[K], pi[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) {
@@ -240,10 +241,20 @@ __device__ __forceinline__ void gmres_lsq_body(const double* __restrict__ rows, 
 }
 
 template <int MB>
-__global__ __launch_bounds__(64) void gmres_lsq_kernel(const double* __restrict__ rows, int ldr, int m, double tol,
-                                                       GmresDevState* st)
+__global__ __launch_bounds__(64) void gmres_lsq_kernel(double* rows, int ldr, int m, double tol, GmresDevState* st,
+                                                       const double* npart, int npn)
 {
-    if (threadIdx.x != 0 || st->skip) return;
+    if (st->skip) {
+        if (npart && threadIdx.x == 0) st->kept = 0;
+        return;
+    }
+    if (npart) {
+        double s = 0.0;
+        for (int q = threadIdx.x; q < npn; q += 64) s += npart[q];
+        s = kb::wave_sum(s);
+        if (threadIdx.x == 0) rows[long(m) * ldr + 2 * m] = s;
+    }
+    if (threadIdx.x != 0) return;
     if constexpr (MB == kMaxBasis) {
         __shared__ Cx T[(MB + 1) * MB];
         __shared__ Cx cs[MB], sn[MB], g[MB + 1], y[MB];
@@ -254,6 +265,7 @@ __global__ __launch_bounds__(64) void gmres_lsq_kernel(const double* __restrict_
         double sig[MB + 1];
         gmres_lsq_body<MB>(rows, ldr, m, tol, st, T, cs, sn, g, y, sig);
     }
+    if (npart && st->hlast <= tol) st->skip = 1;
 }
 
 // out[q] = sum_b part[q*nblk + b] in block order; one block per column q
@@ -418,7 +430,7 @@ hipError_t launch_dots(const cpx<R>* V, long ldv, int k, const cpx<R>* w, long n
 template <typename R>
 hipError_t launch_update(const cpx<R>* V, long ldv, int k, const double* d, const CoefPack& scl, cpx<R>* w,
                          long n, double* part, int nblk, hipStream_t s, const double* nrm, const double* dpart,
-                         double* hrow, const int* skip)
+                         int dnblk, double* hrow, const int* skip)
 {
     if (k < 1) return hipErrorInvalidValue;
     const bool nt = stream_basis<R>(k, n);
@@ -426,10 +438,10 @@ hipError_t launch_update(const cpx<R>* V, long ldv, int k, const double* d, cons
         constexpr int K = decltype(kc)::value;
         if (nt)
             hipLaunchKernelGGL((update_kernel<R, K, true>), dim3(nblk), dim3(KB), 0, s, V, ldv, d, scl, nrm, w, n,
-                               part, dpart, nblk, hrow, skip);
+                               part, dpart, dnblk, hrow, skip);
         else
             hipLaunchKernelGGL((update_kernel<R, K, false>), dim3(nblk), dim3(KB), 0, s, V, ldv, d, scl, nrm, w, n,
-                               part, dpart, nblk, hrow, skip);
+                               part, dpart, dnblk, hrow, skip);
         return hipGetLastError();
     });
 }
@@ -467,15 +479,16 @@ hipError_t launch_gmres_restart(const double* nrm, double tol, GmresDevState* st
     hipLaunchKernelGGL(gmres_restart_kernel, dim3(1), dim3(1), 0, s, nrm, tol, st);
     return hipGetLastError();
 }
-hipError_t launch_gmres_lsq(const double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s)
+hipError_t launch_gmres_lsq(double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s,
+                            const double* npart, int npn)
 {
     if (m < 1 || m >= kMaxBasis) return hipErrorInvalidValue;
     if (m <= 2)
-        hipLaunchKernelGGL(gmres_lsq_kernel<2>, dim3(1), dim3(1), 0, s, rows, ldr, m, tol, st);
+        hipLaunchKernelGGL(gmres_lsq_kernel<2>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st, npart, npn);
     else if (m <= 5)
-        hipLaunchKernelGGL(gmres_lsq_kernel<5>, dim3(1), dim3(1), 0, s, rows, ldr, m, tol, st);
+        hipLaunchKernelGGL(gmres_lsq_kernel<5>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st, npart, npn);
     else
-        hipLaunchKernelGGL(gmres_lsq_kernel<kMaxBasis>, dim3(1), dim3(1), 0, s, rows, ldr, m, tol, st);
+        hipLaunchKernelGGL(gmres_lsq_kernel<kMaxBasis>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st, npart, npn);
     return hipGetLastError();
 }
 
@@ -545,7 +558,7 @@ hipError_t launch_start(const cpx<R>* b, cpx<R>* w, cpx<R>* x, long n, double* p
                                        hipStream_t, const int*);                                            \
     template hipError_t launch_update<R>(const cpx<R>*, long, int, const double*, const CoefPack&, cpx<R>*,  \
                                          long, double*, int, hipStream_t, const double*, const double*,     \
-                                         double*, const int*);                                              \
+                                         int, double*, const int*);                                         \
     template hipError_t launch_combine_dev<R>(const cpx<R>*, long, int, const double*, const int*, cpx<R>*, \
                                               long, int, hipStream_t, const int*);                          \
     template hipError_t launch_combine<R>(const cpx<R>*, long, int, const CoefPack&, cpx<R>*, long, int,    \

@@ -46,19 +46,23 @@ hipError_t launch_dots(const cpx<R>* V, long ldv, int k, const cpx<R>* w, long n
 // a_c = scl.v[c] * (d[2c] + i d[2c+1]); d is device memory.  With nrm (device
 // memory, ||v_c||^2 per slot) the scale is (1 / sqrt(nrm[c]))^2 instead of
 // scl.v[c], so the pass needs nothing from the host.
-// dpart (optional, short columns): the dots partials (nblk per column, 2k
+// dpart (optional, short columns): the dots partials (dnblk per column, 2k
 // columns); each block sums them itself instead of reading d, and block 0
 // writes the 2k sums to hrow.
 template <typename R>
 hipError_t launch_update(const cpx<R>* V, long ldv, int k, const double* d, const CoefPack& scl, cpx<R>* w,
                          long n, double* part, int nblk, hipStream_t s, const double* nrm = nullptr,
-                         const double* dpart = nullptr, double* hrow = nullptr, const int* skip = nullptr);
+                         const double* dpart = nullptr, int dnblk = 0, double* hrow = nullptr,
+                         const int* skip = nullptr);
 constexpr int kInBlockDots = 256;  // dots columns of at most this many partials are summed in the update pass
+// Stencil blocks (and so dots partials per column) up to which the Arnoldi
+// steps of a short vector run as two launches (launch_stencil_step).
+constexpr int kStepBlocks = 768;
 template <typename R>
 hipError_t launch_combine(const cpx<R>* V, long ldv, int k, const CoefPack& a, cpx<R>* x, long n, int nblk,
                           hipStream_t s);
 // x += sum_{c < min(k, *kept)} a_c v_c with a (2k doubles) and kept in
-// device memory.
+// device memory (kept = 0: nothing).
 template <typename R>
 hipError_t launch_combine_dev(const cpx<R>* V, long ldv, int k, const double* a, const int* kept, cpx<R>* x,
                               long n, int nblk, hipStream_t s, const int* skip = nullptr);
@@ -69,7 +73,11 @@ hipError_t launch_combine_dev(const cpx<R>* V, long ldv, int k, const double* a,
 hipError_t launch_gmres_start(const double* nrm, GmresDevState* st, hipStream_t s);
 hipError_t launch_gmres_gate(GmresDevState* st, hipStream_t s);
 hipError_t launch_gmres_restart(const double* nrm, double tol, GmresDevState* st, hipStream_t s);
-hipError_t launch_gmres_lsq(const double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s);
+// npart (optional): ||w_m||^2 is summed from these npn partials first, and a
+// cycle that the state skips leaves kept = 0, so that the combine needs no flag
+// and a stop skips the following cycles' steps.
+hipError_t launch_gmres_lsq(double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s,
+                            const double* npart = nullptr, int npn = 0);
 hipError_t launch_interleave(const double* re, const double* im, cpx<double>* z, long n, hipStream_t s);
 hipError_t launch_deinterleave(const cpx<double>* z, double* re, double* im, long n, hipStream_t s);
 // b = a, c = float(a)

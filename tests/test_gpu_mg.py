@@ -162,3 +162,25 @@ def test_pool_of_hierarchies_matches_single():
     for (xr, ir), x, inf in zip(ref, xs, infos):
         assert inf.converged and inf.iters == ir.iters
         assert float((x - xr).norm() / xr.norm()) <= 1e-12
+
+
+# cycle lengths either side of the longest one whose steps run as two launches
+# (8), a one-step coarse cycle, restarts that the state skips (many cycles)
+@pytest.mark.parametrize("k", [(2, 8, 2, 9), (2, 9, 2, 8), (1, 2, 6, 1), (16, 2, 16, 3)])
+@pytest.mark.parametrize("precision", ["c128", "mixed"])
+def test_mg_cycle_lengths(k, precision):
+    import torch
+    from helm3d.mg import MLGMRES
+    from helm3d.models import config_small, extend, point_source, vec, wavenumber
+    cfg = config_small(n=(22, 19, 17), npml=6, freq=6.0)
+    print(f"cycles k={k} {precision}", flush=True)
+    M = MLGMRES(vec(cfg.v), cfg.n_phys, cfg.h, cfg.npml, cfg.freq, nlevels=3, k=k)
+    b = point_source(cfg, cfg.sources[0])
+    wn = vec(wavenumber(extend(cfg.v, cfg.npml), cfg.freq))
+    h3, p6 = (cfg.h,) * 3, np.array(cfg.npml6)
+    for mode, v in ((1, "forw"), (2, "adj")):
+        x, info = M.solve(torch.from_numpy(b).cuda(), mode=mode, tol=1e-9, precision=precision)
+        r = b - O.hmvp(v, wn, h3, cfg.nt, p6, x.cpu().numpy())
+        assert info.converged and np.linalg.norm(r) < 1e-9 * np.linalg.norm(b)
+        z, iz = M.solve(torch.zeros_like(x), mode=mode, tol=1e-9, precision=precision)
+        assert iz.converged and not z.cpu().numpy().any()
