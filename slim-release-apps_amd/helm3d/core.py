@@ -7,6 +7,7 @@ context's device, x fastest (flattened in MATLAB column-major order).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 from dataclasses import dataclass, field
 from typing import Optional, Sequence
@@ -19,7 +20,12 @@ from ._lib import check, lib
 
 
 def _stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the current stream of the current device (torch.cuda.current_stream()
+    # builds a Stream object for it: 2.7 us of an 11 us call)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+_SAME_DEVICE = contextlib.nullcontext()
 
 
 def _dptr(t: torch.Tensor) -> int:
@@ -89,7 +95,15 @@ class Helm3d:
             pass
 
     def _bind(self):
-        check(lib().helm3d_set_stream(self._ctx, ctypes.c_void_p(_stream_ptr())))
+        check(lib().helm3d_set_stream(self._ctx, _stream_ptr()))
+
+    def _on_device(self):
+        """torch.cuda.device(self.device), or nothing where that device is
+        current already."""
+        index = self.device.index
+        if index is not None and index == torch._C._cuda_getDevice():
+            return _SAME_DEVICE
+        return torch.cuda.device(self.device)
 
     # -- model --------------------------------------------------------------
     def set_model(self, n, h, npml, wn: torch.Tensor):
@@ -105,7 +119,7 @@ class Helm3d:
         n3 = (ctypes.c_int * 3)(*self.n)
         h3 = (ctypes.c_double * 3)(*self.h)
         p6 = (ctypes.c_int * 6)(*self.npml)
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_set_model(self._ctx, n3, h3, p6, ctypes.c_void_p(_dptr(wn)),
                                          int(self.wn_complex)))
@@ -120,10 +134,13 @@ class Helm3d:
     def _vec(self, x: torch.Tensor, dtype) -> torch.Tensor:
         if x.device != self.device:
             raise ValueError(f"vector on {x.device}, operator on {self.device}")
-        x = x.reshape(-1)
+        if x.dim() != 1:
+            x = x.reshape(-1)
         if x.numel() != self.N:
             raise ValueError("vector must have prod(n) elements")
-        return x.to(dtype).contiguous()
+        if x.dtype != dtype:
+            x = x.to(dtype)
+        return x.contiguous()
 
     def apply(self, x: torch.Tensor, adjoint: bool = False, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """y = H x (or H^H x).  complex128 input runs the FP64 kernel, complex64
@@ -132,10 +149,10 @@ class Helm3d:
         dt = torch.complex64 if prec == _lib.HELM3D_C64 else torch.complex128
         x = self._vec(x, dt)
         y = out if out is not None else torch.empty_like(x)
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
-            check(lib().helm3d_apply(self._ctx, _lib.HELM3D_ADJ if adjoint else _lib.HELM3D_FORW, prec,
-                                     ctypes.c_void_p(_dptr(x)), ctypes.c_void_p(_dptr(y))))
+            check(lib().helm3d_apply(self._ctx, _lib.HELM3D_ADJ if adjoint else _lib.HELM3D_FORW, prec, _dptr(x),
+                                     _dptr(y)))
         return y
 
     def apply_deriv(self, dwn: torch.Tensor, x: torch.Tensor, adjoint: bool = False) -> torch.Tensor:
@@ -148,7 +165,7 @@ class Helm3d:
         if dwn.numel() != self.N:
             raise ValueError("dwn must have prod(n) elements")
         y = torch.empty_like(x)
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_apply_deriv(self._ctx, int(adjoint), prec, ctypes.c_void_p(_dptr(dwn)),
                                            ctypes.c_void_p(_dptr(x)), ctypes.c_void_p(_dptr(y))))
@@ -184,7 +201,7 @@ class Helm3d:
         if return_hst:
             cap = int(min(maxit * maxinnerit + 1, 1 << 22))
             hst = np.zeros(cap)
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             code = lib().helm3d_solve(self._ctx, int(mode), ctypes.c_void_p(_dptr(b)), ctypes.c_void_p(_dptr(x)),
                                       ctypes.byref(o), ctypes.byref(info),
@@ -206,7 +223,7 @@ class Helm3d:
         x = torch.zeros_like(b) if x0 is None else self._vec(x0, torch.complex128).clone()
         o = self._opts(tol, maxinnerit, maxit, x0 is not None, inner_tol, inner_m, inner_maxit, inner)
         info = _lib.SolveInfo()
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             code = lib().helm3d_solve_mixed(self._ctx, int(mode), ctypes.c_void_p(_dptr(b)),
                                             ctypes.c_void_p(_dptr(x)), ctypes.byref(o), ctypes.byref(info))
@@ -222,7 +239,7 @@ class Helm3d:
         x = torch.zeros_like(b)
         o = self._opts(tol, 20, maxit, False)
         info = _lib.SolveInfo()
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             code = lib().helm3d_solve_bicgstab(self._ctx, int(mode), ctypes.c_void_p(_dptr(b)),
                                                ctypes.c_void_p(_dptr(x)), ctypes.byref(o), ctypes.byref(info))
@@ -236,7 +253,7 @@ class Helm3d:
         A x = b, A = H (mode 1) or H^H (Helm3dkaczswp_mex.c:60-117)."""
         y = self._vec(x, torch.complex128).clone()
         bb = self._vec(b, torch.complex128) if b is not None else None
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_kacz_sweep(self._ctx, int(mode), float(omega), int(nsweeps),
                                           ctypes.c_void_p(_dptr(y)),
@@ -253,7 +270,7 @@ class Helm3d:
         x = torch.zeros_like(b)
         o = self._opts(tol, 20, maxit, False)
         info = _lib.SolveInfo()
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             code = fn(self._ctx, int(mode), ctypes.c_void_p(_dptr(b)), ctypes.c_void_p(_dptr(x)), ctypes.byref(o),
                       ctypes.byref(info))
@@ -268,13 +285,13 @@ class Helm3d:
 
     def set_graphs(self, enable: bool):
         """Replay fixed kernel sequences from captured HIP graphs (default on)."""
-        with torch.cuda.device(self.device):
+        with self._on_device():
             check(lib().helm3d_set_option(self._ctx, _lib.HELM3D_OPT_GRAPHS, int(enable)))
 
     # -- launch shape ---------------------------------------------------------
     def set_launch(self, kchunk: int = 0, tile_rows: int = 4, prefetch: int = 1, rows_per_thread: int = 1):
         """Stencil launch shape (results are identical for every shape)."""
-        with torch.cuda.device(self.device):
+        with self._on_device():
             check(lib().helm3d_set_launch(self._ctx, int(kchunk), int(tile_rows), int(prefetch),
                                           int(rows_per_thread)))
 
@@ -283,7 +300,7 @@ class Helm3d:
         prec = {"c128": _lib.HELM3D_C128, "c64": _lib.HELM3D_C64}[precision]
         v = [ctypes.c_int(0) for _ in range(4)]
         ms = ctypes.c_double(0)
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_autotune(self._ctx, int(mode), prec, int(reps), *[ctypes.byref(a) for a in v],
                                         ctypes.byref(ms)))
@@ -292,7 +309,7 @@ class Helm3d:
 
     def get_launch(self) -> dict:
         v = [ctypes.c_int(0) for _ in range(5)]
-        with torch.cuda.device(self.device):
+        with self._on_device():
             check(lib().helm3d_get_launch(self._ctx, *[ctypes.byref(a) for a in v]))
         return dict(kchunk=v[0].value, tile_rows=v[1].value, prefetch=v[2].value, rows_per_thread=v[3].value,
                     blocks=v[4].value)
@@ -300,14 +317,14 @@ class Helm3d:
     # -- in-library kernel timing -------------------------------------------
     def profile(self, enable: bool = True):
         """Enable/disable HIP-event timing of every kernel class (resets totals)."""
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_profile(self._ctx, int(enable)))
 
     def profile_read(self) -> dict:
         """{kind: (total_ms, launches)} since the last profile() call."""
         out = {}
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             for name, k in _lib.PROF_KINDS.items():
                 ms = ctypes.c_double(0)
@@ -333,7 +350,7 @@ class Helm3d:
             d = dwn.reshape(-1).to(device=self.device, dtype=torch.float64).contiguous()
             if d.numel() != self.N:
                 raise ValueError("dwn must have prod(n) elements")
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_fwi_grad_accum(self._ctx, ctypes.c_void_p(_dptr(d)) if d is not None else None,
                                               ctypes.c_void_p(_dptr(U)), ctypes.c_void_p(_dptr(V)),
@@ -359,7 +376,7 @@ class Helm3d:
         dwn = torch.empty_like(wn) if derivs >= 1 else None
         ddwn = torch.empty_like(wn) if derivs >= 2 else None
         P = lambda t: ctypes.c_void_p(_dptr(t)) if t is not None else None  # noqa: E731
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_param2wavenum(self._ctx, (ctypes.c_int * 3)(*n_phys), (ctypes.c_int * 6)(*p6),
                                              P(v), _lib.HELM3D_UNITS[unit], float(freq), P(wn), P(dwn), P(ddwn)))
@@ -383,7 +400,7 @@ class Helm3d:
             accumulate = False
         elif g.dtype != torch.float64 or not g.is_contiguous() or g.numel() != int(np.prod(n_phys)):
             raise ValueError("g must be a contiguous float64 tensor on the physical grid")
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_extension_adjoint(self._ctx, (ctypes.c_int * 3)(*n_phys), (ctypes.c_int * 6)(*p6),
                                                  ctypes.c_void_p(_dptr(gpml)), ctypes.c_void_p(_dptr(g)),
@@ -400,7 +417,7 @@ class Helm3d:
             raise ValueError(f"shape mismatch: op {op.shape}, x {x.numel()}, out {out.numel()}")
         if not (x.is_contiguous() and out.is_contiguous()):
             raise ValueError("vectors must be contiguous")
-        with torch.cuda.device(self.device):
+        with self._on_device():
             self._bind()
             check(lib().helm3d_csr_apply(self._ctx, op.nrows, ctypes.c_void_p(_dptr(op.rowptr)),
                                          ctypes.c_void_p(_dptr(op.col)), ctypes.c_void_p(_dptr(op.w)),
