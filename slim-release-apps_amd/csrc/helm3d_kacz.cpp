@@ -170,64 +170,55 @@ int helm3d_solve_cgmn(helm3d_ctx* c, int mode, const void* bv, void* xv, const h
     const double omega = 1.5;  // linearsolve.m:53
     const long N = c->N;
     const long ld = slot_ld(N);
-    CHK(ensure_vecs(c->T64, N, 5));
+    CHK(ensure_vecs(c->T64, N, 4));
     CHK(ensure_work(c));
     cpx<double>* r = c->T64.p;
     cpx<double>* p = r + ld;
-    cpx<double>* Ap = r + 2 * ld;
-    cpx<double>* t = r + 3 * ld;
-    cpx<double>* bp = r + 4 * ld;
+    cpx<double>* t = r + 2 * ld;  // swept copy of p, then A' p
+    cpx<double>* bp = r + 3 * ld;
     const cpx<double>* b = static_cast<const cpx<double>*>(bv);
     cpx<double>* x = static_cast<cpx<double>*>(xv);
     const hipStream_t st = c->stream;
     const int nblk = krylov_blocks(N);
     const cpx<double>* none = nullptr;
-    auto norm2 = [&](const cpx<double>* v, double* out) -> int {
-        HIPCHK(launch_norm2<double>(v, N, c->part, nblk, st));
-        HIPCHK(launch_reduce(c->part, nblk, 1, c->small, st));
-        HIPCHK(hipMemcpyAsync(c->small_host, c->small, sizeof(double), hipMemcpyDeviceToHost, st));
+    // reduced partials land in the pinned mirror
+    const int ub = update_blocks(N);
+    auto fetch = [&](int blocks, int nq) -> int {
+        HIPCHK(launch_reduce(c->part, blocks, nq, c->small, st, c->small_host_dev));
         HIPCHK(hipStreamSynchronize(st));
-        *out = c->small_host[0];
         return HELM3D_OK;
     };
     // b' = SWP(0, b)
     HIPCHK((launch_axpby<double, double>(0.0, 0.0, none, 0.0, 0.0, bp, N, false, st)));
     CHK(sweep(c, mode, omega, bp, b, 1));
-    // x = 0, r = p = b'
+    // x = 0, r = p = t = b'
     HIPCHK((launch_axpby<double, double>(0.0, 0.0, none, 0.0, 0.0, x, N, false, st)));
     HIPCHK((launch_axpby<double, double>(1.0, 0.0, bp, 0.0, 0.0, r, N, false, st)));
     HIPCHK((launch_axpby<double, double>(1.0, 0.0, bp, 0.0, 0.0, p, N, false, st)));
-    double nb2 = 0;
-    CHK(norm2(bp, &nb2));
-    const double normb = std::sqrt(nb2);
+    HIPCHK((launch_axpby<double, double>(1.0, 0.0, bp, 0.0, 0.0, t, N, false, st)));
+    HIPCHK(launch_norm2<double>(bp, N, c->part, nblk, st));
+    CHK(fetch(nblk, 1));
+    const double normb = std::sqrt(c->small_host[0]);
     double normr = normb;
     long k = 0;
     double rel = normb > 0 ? 1.0 : 0.0;
     if (normb > 0) {
         while (true) {
-            // Ap = p - SWP(p, 0)
-            HIPCHK((launch_axpby<double, double>(1.0, 0.0, p, 0.0, 0.0, t, N, false, st)));
+            // Ap = p - SWP(p, 0), in t (which holds p); pAp = p^H Ap
             CHK(sweep(c, mode, omega, t, nullptr, 1));
-            HIPCHK((launch_axpby<double, double>(1.0, 0.0, p, -1.0, 0.0, t, N, true, st)));
-            std::swap(Ap, t);
-            // pAp = p^H Ap
-            HIPCHK(launch_dots<double>(p, ld, 1, Ap, N, c->part, nblk, st));
-            HIPCHK(launch_reduce(c->part, nblk, 2, c->small, st));
-            HIPCHK(hipMemcpyAsync(c->small_host, c->small, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            HIPCHK(launch_cg_apply(p, t, N, c->part, st));
+            CHK(fetch(ub, 2));
             const std::complex<double> pAp(c->small_host[0], c->small_host[1]);
             const std::complex<double> alpha = (normr * normr) / pAp;
-            HIPCHK((launch_axpby<double, double>(alpha.real(), alpha.imag(), p, 1.0, 0.0, x, N, true, st)));
-            HIPCHK((launch_axpby<double, double>(-alpha.real(), -alpha.imag(), Ap, 1.0, 0.0, r, N, true, st)));
+            HIPCHK(launch_cg_step(alpha.real(), alpha.imag(), p, t, x, r, nullptr, N, c->part, st));
             const double normr_old = normr;
-            double nr2 = 0;
-            CHK(norm2(r, &nr2));
-            normr = std::sqrt(nr2);
+            CHK(fetch(ub, 1));
+            normr = std::sqrt(c->small_host[0]);
             rel = normr / normb;
             ++k;
             if (k >= o.maxit || !(rel > o.tol)) break;  // CGMN.m: stop at hst(end) <= tol
             const double beta = (normr / normr_old) * (normr / normr_old);
-            HIPCHK((launch_axpby<double, double>(1.0, 0.0, r, beta, 0.0, p, N, true, st)));
+            HIPCHK(launch_cg_dir(r, beta, p, t, N, st));
         }
     } else {
         HIPCHK((launch_axpby<double, double>(0.0, 0.0, none, 0.0, 0.0, x, N, false, st)));
@@ -262,6 +253,12 @@ int helm3d_solve_crmn(helm3d_ctx* c, int mode, const void* bv, void* xv, const h
     // host copies of a few reduced values
     auto fetch = [&](int count) -> int {
         HIPCHK(hipMemcpyAsync(c->small_host, c->small, count * sizeof(double), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        return HELM3D_OK;
+    };
+    // reduced partials of the update passes land in the pinned mirror
+    auto fetch_part = [&](int nq) -> int {
+        HIPCHK(launch_reduce(c->part, update_blocks(N), nq, c->small, st, c->small_host_dev));
         HIPCHK(hipStreamSynchronize(st));
         return HELM3D_OK;
     };
@@ -301,27 +298,20 @@ int helm3d_solve_crmn(helm3d_ctx* c, int mode, const void* bv, void* xv, const h
         while (true) {
             // CRMN.m:68-88
             const std::complex<double> gamma = rAr / nAp2;
-            HIPCHK((launch_axpby<double, double>(gamma.real(), gamma.imag(), p, 1.0, 0.0, x, N, true, st)));
-            HIPCHK((launch_axpby<double, double>(-gamma.real(), -gamma.imag(), Ap, 1.0, 0.0, r, N, true, st)));
-            HIPCHK(launch_norm2<double>(r, N, c->part, nblk, st));
-            HIPCHK(launch_reduce(c->part, nblk, 1, c->small, st));
-            CHK(fetch(1));
+            HIPCHK(launch_cg_step(gamma.real(), gamma.imag(), p, Ap, x, r, Ar, N, c->part, st));
+            CHK(fetch_part(1));
             rel = std::sqrt(c->small_host[0]) / normb;
             ++k;
             if (k >= o.maxit || !(rel > o.tol)) break;  // stop at hst(end) <= tol
-            // CRMN.m:94-106
-            CHK(apply(r, Ar));
-            HIPCHK(launch_dots<double>(r, ld, 1, Ar, N, c->part, nblk, st));
-            HIPCHK(launch_reduce(c->part, nblk, 2, c->small, st));
-            CHK(fetch(2));
+            // CRMN.m:94-106; Ar holds r
+            CHK(sweep(c, mode, omega, Ar, nullptr, 1));
+            HIPCHK(launch_cg_apply(r, Ar, N, c->part, st));
+            CHK(fetch_part(2));
             const std::complex<double> old = rAr;
             rAr = std::complex<double>(c->small_host[0], c->small_host[1]);
             const std::complex<double> beta = rAr / old;
-            HIPCHK((launch_axpby<double, double>(1.0, 0.0, r, beta.real(), beta.imag(), p, N, true, st)));
-            HIPCHK((launch_axpby<double, double>(1.0, 0.0, Ar, beta.real(), beta.imag(), Ap, N, true, st)));
-            HIPCHK(launch_norm2<double>(Ap, N, c->part, nblk, st));
-            HIPCHK(launch_reduce(c->part, nblk, 1, c->small, st));
-            CHK(fetch(1));
+            HIPCHK(launch_cr_dir(r, beta.real(), beta.imag(), p, Ar, Ap, N, c->part, st));
+            CHK(fetch_part(1));
             nAp2 = c->small_host[0];
         }
     }

@@ -91,6 +91,17 @@ hipError_t launch_axpby(double ar, double ai, const cpx<RX>* x, double br, doubl
                         bool use_y, hipStream_t s);
 template <typename R>
 hipError_t launch_norm2(const cpx<R>* x, long n, double* part, int nblk, hipStream_t s);
+// CGMN / CRMN vector passes; partials of update_blocks(n) blocks.
+// p = r + beta p, t = p
+hipError_t launch_cg_dir(const cpx<double>* r, double beta, cpx<double>* p, cpx<double>* t, long n, hipStream_t s);
+// p = r + beta p, ap = ar + beta ap, partial ||ap||^2
+hipError_t launch_cr_dir(const cpx<double>* r, double br, double bi, cpx<double>* p, const cpx<double>* ar,
+                         cpx<double>* ap, long n, double* part, hipStream_t s);
+// t = p - t, partials of p^H t (two columns)
+hipError_t launch_cg_apply(const cpx<double>* p, cpx<double>* t, long n, double* part, hipStream_t s);
+// x += a p, r -= a ap, partial ||r||^2; copy (optional) = r
+hipError_t launch_cg_step(double ar, double ai, const cpx<double>* p, const cpx<double>* ap, cpx<double>* x,
+                          cpx<double>* r, cpx<double>* copy, long n, double* part, hipStream_t s);
 // w = b, x = 0 and the partials of ||b||^2 (those of launch_norm2 on w) in one pass.
 template <typename R>
 hipError_t launch_start(const cpx<R>* b, cpx<R>* w, cpx<R>* x, long n, double* part, int nblk, hipStream_t s);
