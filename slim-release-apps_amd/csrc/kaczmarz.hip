@@ -178,7 +178,7 @@ __global__ __launch_bounds__(KB) void kacz_color_kernel(OpDesc<double> op, doubl
 // 407 and 134 / 122 us.  Eight lanes per row: 1.95 / 1.95 ms, 212 / 199 and
 // 122 / 117 us (more instructions in all); two: spills.
 constexpr int kLineThreads = 512;      // largest block
-constexpr size_t kLineLds = 64 * 1024;  // LDS of a block
+constexpr size_t kLineLds = 159 * 1024;  // LDS of a block (one kilobyte short of all of it)
 
 struct LineCoef {
     cpx<double> K;
@@ -455,8 +455,9 @@ hipError_t launch_line(const OpDesc<double>& op, double omega, cpx<double>* x, c
 }  // namespace
 
 // nsweeps double sweeps: colours 0 .. 26 and back.  The line form runs while
-// its nine lines fit in LDS (nx up to 299 forward, 449 adjoint, 224 forward
-// with complex wn); longer lines take a launch per colour.
+// its nine lines fit in LDS (nx up to 747 forward, 1122 adjoint, 560 forward
+// with complex wn), also where a compute unit holds one block only (740 x 80 x
+// 60 forward 0.90 ms, by colours 2.21); longer lines take a launch per colour.
 hipError_t launch_kacz_sweep(bool adj, const OpDesc<double>& op, double omega, cpx<double>* x,
                              const cpx<double>* b, int nsweeps, hipStream_t s)
 {

@@ -204,3 +204,11 @@ def test_device_sweep_line_lengths(n, variant):
     y = H.kacz_sweep(torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda(), mode=mode, nsweeps=2).cpu().numpy()
     yo = O.kacz_sweep(variant, wn, h, n, npml, 1.5, O.kacz_sweep(variant, wn, h, n, npml, 1.5, x, b), b)
     assert relerr(y, yo) <= 1e-12
+
+
+# either side of the longest line that fits in LDS at all (747 points forward,
+# 1122 adjoint, 560 forward with complex wn)
+@pytest.mark.parametrize("nx,variant", [(747, "forw"), (748, "forw"), (1122, "adj"), (1123, "adj"), (560, "forw_wnc"),
+                                        (561, "forw_wnc"), (1122, "adj_wnc")])
+def test_device_sweep_longest_lines(nx, variant):
+    test_device_sweep_line_lengths((nx, 4, 3), variant)
