@@ -146,6 +146,9 @@ struct helm3d_ctx {
     // one shape for both
     StencilGrid grid{}, grid32{};
     bool grid_auto = true;
+    // the shapes by rule, kept for launches whose block sums reach the result
+    // (the Arnoldi steps of short vectors): their bits follow the grid alone
+    StencilGrid rule64{}, rule32{};
 
     double* part = nullptr;
     size_t part_cap = 0;
@@ -276,6 +279,12 @@ inline const StencilGrid& grid_of(const helm3d_ctx* c)
     if constexpr (std::is_same<R, double>::value) return c->grid;
     else return c->grid32;
 }
+template <typename R>
+inline const StencilGrid& rule_of(const helm3d_ctx* c)
+{
+    if constexpr (std::is_same<R, double>::value) return c->rule64;
+    else return c->rule32;
+}
 
 inline int bind(helm3d_ctx* c)
 {
@@ -329,7 +338,8 @@ constexpr long kMaxDeviceCycles = 16;
 // mirror) and the stencil's write-only sink.
 inline int ensure_work(helm3d_ctx* c)
 {
-    const size_t nblk = std::max<size_t>(std::max(c->grid.blocks, c->grid32.blocks), kMaxPartials);
+    const size_t nblk = std::max<size_t>(
+        std::max(std::max(c->grid.blocks, c->grid32.blocks), std::max(c->rule64.blocks, c->rule32.blocks)), kMaxPartials);
     CHK(ensure_t(&c->part, &c->part_cap, nblk * 2 * kMaxBasis));
     CHK(ensure_t(&c->small, &c->small_cap, 2 * kMaxBasis + 8));
     CHK(ensure(&c->sink, &c->sink_cap, size_t(kSinkSlots) * sizeof(cpx<double>)));

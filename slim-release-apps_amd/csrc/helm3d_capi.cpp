@@ -93,7 +93,7 @@ Vecs<float>& zbasis_of<float>(helm3d_ctx* c) { return c->Z32; }
 // Stencil launch on the context's operator; y = alpha*Hx + beta*b.
 template <typename R>
 int stencil(helm3d_ctx* c, int variant, const OpDesc<R>& op, const cpx<R>* x, cpx<R>* y, R alpha,
-            const cpx<R>* b, R beta, double* norm_part, const int* skip = nullptr)
+            const cpx<R>* b, R beta, double* norm_part, const int* skip = nullptr, const StencilGrid* shape = nullptr)
 {
     StencilLaunch<R> L{};
     L.skip = skip;
@@ -105,7 +105,7 @@ int stencil(helm3d_ctx* c, int variant, const OpDesc<R>& op, const cpx<R>* x, cp
     L.beta = beta;
     L.norm_part = norm_part;
     L.sink = static_cast<cpx<R>*>(c->sink);
-    TIMED(HELM3D_PROF_STENCIL, launch_stencil<R>(variant, L, grid_of<R>(c), c->stream));
+    TIMED(HELM3D_PROF_STENCIL, launch_stencil<R>(variant, L, shape ? *shape : grid_of<R>(c), c->stream));
     return HELM3D_OK;
 }
 
@@ -237,7 +237,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
     // (or the start) left of its input's norm, the update pass the dots; the
     // first step of a cycle takes the stop decisions, the least squares the
     // norm of the last slot.  Partials: norms at the front, dots behind them.
-    const StencilGrid& G = grid_of<R>(c);
+    const StencilGrid& G = rule_of<R>(c);
     if (device_driven && nblk <= kInBlockDots && G.blocks <= kStepBlocks && m <= kStepMaxK) {
         double* dpart = c->part + kStepBlocks;
         auto steps = [&](hipStream_t s, int start, int npn) -> int {
@@ -271,7 +271,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
         };
         for (long cyc = 0; (1 + cyc * long(m)) / m < maxit; ++cyc) {
             const bool resid = cyc > 0 || use_x0;
-            if (resid) CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, cyc > 0 ? skip : nullptr));
+            if (resid) CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, cyc > 0 ? skip : nullptr, &G));
             else HIPCHK(launch_start<R>(b, slot(0), x, N, c->part, nblk, c->stream));
             const int start = cyc > 0 ? 2 : 1, npn = resid ? G.blocks : nblk;
             if (c->use_graphs && !c->prof)
@@ -868,8 +868,8 @@ int helm3d_set_model(helm3d_ctx* c, const int n[3], const double h[3], const int
     fill_opdesc(c->op64, n, c->hc, c->tab64, off, c->wn64, c->wnc, ilo, ihi);
     fill_opdesc(c->op32, n, c->hc, c->tab32, off, c->wn32, c->wnc, ilo, ihi);
     if (!same_grid) {
-        c->grid = stencil_grid<double>(n[0], n[1], n[2], 0);
-        c->grid32 = stencil_grid<float>(n[0], n[1], n[2], 0);
+        c->grid = c->rule64 = stencil_grid<double>(n[0], n[1], n[2], 0);
+        c->grid32 = c->rule32 = stencil_grid<float>(n[0], n[1], n[2], 0);
         c->grid_auto = true;
     }
     CHK(ensure_work(c));
