@@ -180,14 +180,11 @@ struct helm3d_ctx {
     double* bsc = nullptr;  // BiCGStab device scalars (BS_SLOTS doubles)
     size_t bsc_cap = 0;
 
-    // captured Arnoldi cycles of the unpreconditioned GMRES on small grids:
-    // cyc_graph[p + 2 w] for precision p (0: complex128, 1: complex64) and
-    // w = 0 the host-driven cycle (and the device-driven one of four launches a
-    // step), the device-driven cycle of two launches a step opened from x = 0
-    // (1), from a given x (2) or by a restart (3); with the bytes of the launch
-    // arguments they were captured with (a different key recaptures)
-    hipGraphExec_t cyc_graph[8] = {};
-    std::vector<unsigned char> cyc_key[8];
+    // captured Arnoldi cycle of the unpreconditioned GMRES on small grids,
+    // one per precision (0: complex128, 1: complex64), with the bytes of the
+    // launch arguments it was captured with (a different key recaptures)
+    hipGraphExec_t cyc_graph[2] = {nullptr, nullptr};
+    std::vector<unsigned char> cyc_key[2];
 
     // captured fixed-length complex64 inner solve (mixed precision)
     hipStream_t cap_stream = nullptr;

@@ -50,9 +50,10 @@ struct StencilLaunch {
 
 struct GmresDevState;
 
-// Arnoldi step of the device-driven GMRES on small grids (EPI 5): y = H x /
+// Arnoldi step of GMRES on small grids (EPI 5): y = H x /
 // ||x||, then the dots of y with the basis slots, in one launch.
 //   npart, npn  partial sums of ||x||^2, added by every wave in one order
+//               (npart = nullptr: y = H x, and the fields up to tol unused)
 //   nrm, row    ||x||^2 stored by block 0 for the update pass and the least
 //               squares (row optional)
 //   start       0: an inner step; 1: first step of a solve, 2: of a restarted

@@ -289,7 +289,7 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     for (int r = 0; r < RY; ++r) Xlast[r] = Rlast[r] = Dlast[r] = zero<R>();
     // output scale: alpha, or alpha / sqrt(*anrm) with the norm held on the device
     R alpha = (EPI <= 1 && L.anrm) ? R(double(L.alpha) / sqrt(*L.anrm)) : L.alpha;
-    if constexpr (EPI == 5) {
+    if (EPI == 5 && X->npart) {
         // every wave adds the partials of ||x||^2 in the same order
         double s = 0.0;
         for (int q = tx; q < X->npn; q += 64) s += X->npart[q];

@@ -134,9 +134,9 @@ namespace helm3d {
 // shape, cycle length and every buffer address the steps use.
 template <typename R, typename Rec>
 int cycle_graph(helm3d_ctx* c, int variant, int m, const cpx<R>* V, long ld, int nblk, const int* skip,
-                Rec&& record, int which = 0, double tol = 0.0)
+                Rec&& record)
 {
-    const int p = (std::is_same<R, double>::value ? 0 : 1) + 2 * which;
+    const int p = (std::is_same<R, double>::value ? 0 : 1) ;
     std::vector<unsigned char> key;
     auto put = [&](const void* a, size_t n) {
         const auto* b = static_cast<const unsigned char*>(a);
@@ -149,7 +149,6 @@ int cycle_graph(helm3d_ctx* c, int variant, int m, const cpx<R>* V, long ld, int
     put(&op, sizeof(op));
     put(ptrs, sizeof(ptrs));
     put(ints, sizeof(ints));
-    put(&tol, sizeof(tol));
     if (!c->cyc_graph[p] || c->cyc_key[p] != key) {
         if (c->cyc_graph[p]) {
             HIPCHK(hipGraphExecDestroy(c->cyc_graph[p]));
@@ -237,8 +236,11 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
     // (or the start) left of its input's norm, the update pass the dots; the
     // first step of a cycle takes the stop decisions, the least squares the
     // norm of the last slot.  Partials: norms at the front, dots behind them.
+    // Launched one by one: as captured graphs the short cycles took 3 to 5 %
+    // longer, alone and with four hierarchies at once.
     const StencilGrid& G = rule_of<R>(c);
-    if (device_driven && nblk <= kInBlockDots && G.blocks <= kStepBlocks && m <= kStepMaxK) {
+    const bool short_vecs = nblk <= kInBlockDots && G.blocks <= kStepBlocks;
+    if (device_driven && short_vecs && m <= kStepMaxK) {
         double* dpart = c->part + kStepBlocks;
         auto steps = [&](hipStream_t s, int start, int npn) -> int {
             for (int j = 1; j <= m; ++j) {
@@ -274,12 +276,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
             if (resid) CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, cyc > 0 ? skip : nullptr, &G));
             else HIPCHK(launch_start<R>(b, slot(0), x, N, c->part, nblk, c->stream));
             const int start = cyc > 0 ? 2 : 1, npn = resid ? G.blocks : nblk;
-            if (c->use_graphs && !c->prof)
-                CHK(cycle_graph<R>(c, variant, m, V, ld, npn, skip,
-                                   [&](hipStream_t s) { return steps(s, start, npn); },
-                                   cyc > 0 ? 3 : (resid ? 2 : 1), tol));
-            else
-                CHK(steps(c->stream, start, npn));
+            CHK(steps(c->stream, start, npn));
             TIMED(HELM3D_PROF_COMBINE,
                   launch_combine_dev<R>(V, ld, m, st->coef, &st->kept, x, N, nblk_u, c->stream, nullptr));
         }
@@ -450,18 +447,37 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
         }
         while (P && k <= m && hlast > tol) {
             // w = A z_k into slot k
-            {
-                CHK(P->apply(slot(k - 1), sig[k - 1], Z + size_t(k - 1) * ld));
-                CHK(stencil<R>(c, variant, op, Z + size_t(k - 1) * ld, slot(k), R(1), nullptr, R(0), nullptr));
-            }
+            CHK(P->apply(slot(k - 1), sig[k - 1], Z + size_t(k - 1) * ld));
             // classical Gram-Schmidt, FGMRES.m:100-103; d (2k values) and
             // ||w||^2 reach c->small and its pinned mirror
             CoefPack scl{};
             for (int q = 0; q < k; ++q) scl.v[q] = sig[q] * sig[q];
-            TIMED(HELM3D_PROF_DOTS, launch_dots<R>(V, ld, k, slot(k), N, c->part, nblk_d, c->stream));
-            TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, nblk_d, 2 * k, c->small, c->stream, c->small_host_dev));
-            TIMED(HELM3D_PROF_UPDATE,
-                  launch_update<R>(V, ld, k, c->small, scl, slot(k), N, c->part, nblk_u, c->stream));
+            if (short_vecs && k <= kStepMaxK) {
+                // short vectors: matvec and dots in one launch, the dots
+                // summed by the update pass (three launches instead of five)
+                StencilLaunch<R> L{};
+                L.op = op;
+                L.x = Z + size_t(k - 1) * ld;
+                L.y = slot(k);
+                L.alpha = R(1);
+                L.sink = static_cast<cpx<R>*>(c->sink);
+                StepArgs<R> X{};
+                X.V = V;
+                X.ldv = ld;
+                X.k = k;
+                X.dpart = c->part + kStepBlocks;
+                TIMED(HELM3D_PROF_STENCIL, launch_stencil_step<R>(variant, L, X, G, c->stream));
+                TIMED(HELM3D_PROF_UPDATE,
+                      launch_update<R>(V, ld, k, nullptr, scl, slot(k), N, c->part, nblk, c->stream, nullptr,
+                                       X.dpart, G.blocks, c->small_host_dev));
+            } else {
+                CHK(stencil<R>(c, variant, op, Z + size_t(k - 1) * ld, slot(k), R(1), nullptr, R(0), nullptr));
+                TIMED(HELM3D_PROF_DOTS, launch_dots<R>(V, ld, k, slot(k), N, c->part, nblk_d, c->stream));
+                TIMED(HELM3D_PROF_REDUCE,
+                      launch_reduce(c->part, nblk_d, 2 * k, c->small, c->stream, c->small_host_dev));
+                TIMED(HELM3D_PROF_UPDATE,
+                      launch_update<R>(V, ld, k, c->small, scl, slot(k), N, c->part, nblk_u, c->stream));
+            }
             TIMED(HELM3D_PROF_REDUCE,
                   launch_reduce(c->part, nblk_u, 1, c->small + 2 * k, c->stream, c->small_host_dev + 2 * k));
             HIPCHK(hipStreamSynchronize(c->stream));
