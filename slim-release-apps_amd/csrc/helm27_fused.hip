@@ -7,27 +7,21 @@ namespace helm3d {
 
 namespace {
 
-template <bool ADJ, bool WNC, int TY, int PF, int EPI, int RY>
-__global__ __launch_bounds__(TX* TY / RY) void helm27_fused_kernel(StencilLaunch<float> L)
+// One shape, the one stencil_grid picks by rule: the block sums group the dots
+// by the launch's blocks, so a shape tuned per handle would give two handles of
+// one grid different inner solves.
+constexpr int kFTy = 4, kFPf = 2;
+
+template <bool ADJ, bool WNC, int EPI>
+__global__ __launch_bounds__(TX* kFTy) void helm27_fused_kernel(StencilLaunch<float> L)
 {
-    helm27_body<float, ADJ, false, WNC, TY, PF, EPI, RY>(L, blockIdx.x, gridDim.x);
+    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1>(L, blockIdx.x, gridDim.x);
 }
 
 template <bool A, bool W, int EPI>
 hipError_t launch_shape(const StencilLaunch<float>& L, const StencilGrid& g, hipStream_t s)
 {
-    const dim3 grid(g.blocks);
-    const bool two = g.pf >= 2;  // planes in flight: the four vectors of epilogue 3 leave registers for two
-    if (g.ty == 8 && g.ry == 2) {
-        if (two) hipLaunchKernelGGL((helm27_fused_kernel<A, W, 8, 2, EPI, 2>), grid, dim3(TX * 4), 0, s, L);
-        else hipLaunchKernelGGL((helm27_fused_kernel<A, W, 8, 1, EPI, 2>), grid, dim3(TX * 4), 0, s, L);
-    } else if (g.ty == 8) {
-        if (two) hipLaunchKernelGGL((helm27_fused_kernel<A, W, 8, 2, EPI, 1>), grid, dim3(TX * 8), 0, s, L);
-        else hipLaunchKernelGGL((helm27_fused_kernel<A, W, 8, 1, EPI, 1>), grid, dim3(TX * 8), 0, s, L);
-    } else {
-        if (two) hipLaunchKernelGGL((helm27_fused_kernel<A, W, 4, 2, EPI, 1>), grid, dim3(TX * 4), 0, s, L);
-        else hipLaunchKernelGGL((helm27_fused_kernel<A, W, 4, 1, EPI, 1>), grid, dim3(TX * 4), 0, s, L);
-    }
+    hipLaunchKernelGGL((helm27_fused_kernel<A, W, EPI>), dim3(g.blocks), dim3(TX * kFTy), 0, s, L);
     return hipGetLastError();
 }
 
@@ -39,7 +33,8 @@ hipError_t launch_stencil_fused(int variant, int epi, StencilLaunch<float> L, co
     L.tiles_y = g.tiles_y;
     L.kchunk = g.kchunk;
     const bool adj = variant & VAR_ADJ, wnc = variant & VAR_WNC;
-    if ((variant & VAR_DERIV) || (epi != 3 && epi != 4)) return hipErrorInvalidValue;
+    if ((variant & VAR_DERIV) || (epi != 3 && epi != 4) || g.ty != kFTy || g.ry != 1)
+        return hipErrorInvalidValue;
     if (epi == 3) {
         if (!adj && !wnc) return launch_shape<false, false, 3>(L, g, s);
         if (!adj) return launch_shape<false, true, 3>(L, g, s);

@@ -9,28 +9,20 @@ namespace helm3d {
 
 namespace {
 
-template <typename R, bool ADJ, bool WNC, int TY, int PF, int RY>
-__global__ __launch_bounds__(TX* TY / RY) void helm27_step_kernel(StencilLaunch<R> L, StepArgs<R> X)
+// One shape, the one stencil_grid picks by rule: the dots are grouped by the
+// launch's blocks, and their bits must follow the grid alone.
+constexpr int kSTy = 4, kSPf = 2;
+
+template <typename R, bool ADJ, bool WNC>
+__global__ __launch_bounds__(TX* kSTy) void helm27_step_kernel(StencilLaunch<R> L, StepArgs<R> X)
 {
-    helm27_body<R, ADJ, false, WNC, TY, PF, 5, RY>(L, blockIdx.x, gridDim.x, &X);
+    helm27_body<R, ADJ, false, WNC, kSTy, kSPf, 5, 1>(L, blockIdx.x, gridDim.x, &X);
 }
 
-// one or two planes in flight: the small grids march a few planes per block
 template <typename R, bool A, bool W>
 hipError_t launch_shape(const StencilLaunch<R>& L, const StepArgs<R>& X, const StencilGrid& g, hipStream_t s)
 {
-    const dim3 grid(g.blocks);
-    const bool two = g.pf >= 2;
-    if (g.ty == 8 && g.ry == 2) {
-        if (two) hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 2, 2>), grid, dim3(TX * 4), 0, s, L, X);
-        else hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 1, 2>), grid, dim3(TX * 4), 0, s, L, X);
-    } else if (g.ty == 8) {
-        if (two) hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 2, 1>), grid, dim3(TX * 8), 0, s, L, X);
-        else hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 8, 1, 1>), grid, dim3(TX * 8), 0, s, L, X);
-    } else {
-        if (two) hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 4, 2, 1>), grid, dim3(TX * 4), 0, s, L, X);
-        else hipLaunchKernelGGL((helm27_step_kernel<R, A, W, 4, 1, 1>), grid, dim3(TX * 4), 0, s, L, X);
-    }
+    hipLaunchKernelGGL((helm27_step_kernel<R, A, W>), dim3(g.blocks), dim3(TX * kSTy), 0, s, L, X);
     return hipGetLastError();
 }
 
@@ -43,7 +35,8 @@ hipError_t launch_stencil_step(int variant, StencilLaunch<R> L, const StepArgs<R
     L.tiles_x = g.tiles_x;
     L.tiles_y = g.tiles_y;
     L.kchunk = g.kchunk;
-    if ((variant & VAR_DERIV) || X.k < 1 || X.k > kStepMaxK) return hipErrorInvalidValue;
+    if ((variant & VAR_DERIV) || X.k < 1 || X.k > kStepMaxK || g.ty != kSTy || g.ry != 1)
+        return hipErrorInvalidValue;
     const bool adj = variant & VAR_ADJ, wnc = variant & VAR_WNC;
     if (!adj && !wnc) return launch_shape<R, false, false>(L, X, g, s);
     if (!adj) return launch_shape<R, false, true>(L, X, g, s);
