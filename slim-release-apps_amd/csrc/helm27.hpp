@@ -45,6 +45,7 @@ struct StencilLaunch {
     const cpx<R>* rh;
     double* sc;
     int rho_new, rho_old, first;
+    int narrow;       // work lists: tiles_x counts tiles of 32 columns
     const int* skip;  // optional (device): the launch does nothing while *skip != 0
 };
 
@@ -83,7 +84,7 @@ struct StepArgs {
 constexpr int kSinkSlots = 65536;
 
 struct StencilGrid {
-    int tiles_x, tiles_y, kchunk, nchunks, blocks, ty, pf, ry;
+    int tiles_x, tiles_y, kchunk, nchunks, blocks, ty, pf, ry, tx;
 };
 
 // z planes per block (even) for a launch over columns of `tiles[i]` tiles and
@@ -106,7 +107,8 @@ constexpr int kSlots64 = 512, kSlots32 = 1024;
 // kchunk <= 0 picks the chunk by stencil_chunk for precision R; ty in {4, 8};
 // pf in 1..4; ry in {1, 2} (2 needs ty = 8; otherwise 1 is used).
 template <typename R>
-StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 4, int pf = 2, int ry = 1);
+StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 4, int pf = 2, int ry = 1,
+                         int tx = 64);
 
 template <typename R>
 hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g, hipStream_t s);
@@ -124,9 +126,11 @@ hipError_t launch_stencil_fused(int variant, int epi, StencilLaunch<float> L, co
 // launched with its own tiles_x/tiles_y/kchunk and the common shape (ty, pf,
 // ry: two rows per thread with ty = 8).
 // epi: 0 (y = alpha H x), 1 (+ beta b), 3, 4 (fused BiCGStab forms).
+// mix: items with narrow set have tiles of 32 columns by 8 rows (the others
+// ty x 64, ty = 4, pf = 2, ry = 1).
 // active (nullable): items with active[it] == 0 do nothing.
 template <typename R>
 hipError_t launch_stencil_batch(int variant, int epi, const StencilLaunch<R>* items, const int* first, int nitems,
-                                int blocks, const int* active, int ty, int pf, hipStream_t s, int ry = 1);
+                                int blocks, const int* active, int ty, int pf, hipStream_t s, int ry = 1, bool mix = false);
 
 }  // namespace helm3d

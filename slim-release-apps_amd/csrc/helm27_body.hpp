@@ -19,7 +19,8 @@
 // The adjoint is the exact conjugate transpose: F/G take the neighbour's x/y
 // PML values and the z weights come from the neighbouring planes.
 //
-// Tiling.  A block of 64 x TY / RY threads owns a 64 x TY column tile and
+// Tiling.  A block of TXW x TY / RY threads owns a TXW x TY column tile (TXW =
+// 64, a row per wave, or 32, two rows per wave) and
 // marches over a z chunk.  Each plane (with a one-point x/y halo) is staged
 // once in LDS (double-buffered, one barrier per plane); the loads of the
 // planes ahead are issued before the barrier so HBM latency overlaps the
@@ -39,7 +40,6 @@ namespace helm3d {
 namespace {
 
 constexpr int TX = 64;  // one wavefront along x
-constexpr int HX = TX + 2;
 constexpr int kMaxChunk = 254;  // z planes per block (LDS holds their PML weights)
 
 template <typename R>
@@ -102,14 +102,15 @@ __device__ inline Cd cd_div(Cd a, Cd b)
 // 5 is an Arnoldi step (StepArgs X): EPI 0 with the scale summed from partials
 // and, after the march, the dots of the block's outputs with the basis.
 // The body runs one block `lin` of a launch of `G` blocks described by L.
-template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY = 1>
+template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY = 1, int TXW = TX>
 __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int lin, const int G,
                                             const StepArgs<R>* X = nullptr)
 {
     static_assert(RY == 1 || RY == 2, "one or two rows per thread");
     static_assert(TY % RY == 0, "rows per thread divide the tile rows");
-    constexpr int NT = TX * TY / RY;     // threads
-    constexpr int HY = TY + 2;
+    static_assert(TXW == 64 || TXW == 32, "a wave is one or two rows of the tile");
+    constexpr int NT = TXW * TY / RY;    // threads
+    constexpr int HX = TXW + 2, HY = TY + 2;
     constexpr int NS = HX * HY;          // halo tile slots
     constexpr int NSL = (NS + NT - 1) / NT;  // load slots per thread
     static_assert(PF >= 1 && PF <= 4, "prefetch depth 1 to 4");
@@ -138,13 +139,13 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     const int chunk = logical / ntile;
     const int tile = logical - chunk * ntile;
     const int tyt = tile / L.tiles_x;
-    const int i0 = (tile - tyt * L.tiles_x) * TX;
+    const int i0 = (tile - tyt * L.tiles_x) * TXW;
     const int j0 = tyt * TY;
     const int k0 = chunk * L.kchunk;
     const int k1 = min(nz, k0 + L.kchunk);
 
     const int tid = threadIdx.x;
-    const int tx = tid & (TX - 1), tw = tid / TX;  // lane, wave
+    const int tx = tid & (TXW - 1), tw = tid / TXW;  // tile column, row group (TXW = 64: lane, wave)
     const int tr0 = tw * RY;                       // first tile row of this thread
     const int i = i0 + tx;
     const int ic = min(i, nx - 1);  // clamped for table reads
@@ -153,8 +154,8 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     // launch shape): interior when every column and the row have
     // xi_lo = xi_hi = 1 at index-1, index, index+1, the general path
     // otherwise.
-    const int jw = __builtin_amdgcn_readfirstlane(j0 + tr0);
-    const bool xint = i0 >= op.int_lo[0] && i0 + TX - 1 <= op.int_hi[0];
+    const int jw = TXW == 64 ? __builtin_amdgcn_readfirstlane(j0 + tr0) : j0 + tr0;
+    const bool xint = i0 >= op.int_lo[0] && i0 + TXW - 1 <= op.int_hi[0];
     bool yint[RY], active[RY];
     long offc[RY];
 #pragma unroll
@@ -292,7 +293,7 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     if (EPI == 5 && X->npart) {
         // every wave adds the partials of ||x||^2 in the same order
         double s = 0.0;
-        for (int q = tx; q < X->npn; q += 64) s += X->npart[q];
+        for (int q = tid & 63; q < X->npn; q += 64) s += X->npart[q];
         s = kb::wave_sum(s);
         bool stop = false;
         if (X->start) {
@@ -698,8 +699,8 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
         }
         __shared__ double dred[NT / 64][2 * kStepMaxK];
         int q;
-        const double s = kb::wave_sums<2 * kStepMaxK>(da, tx, q);
-        if (q >= 0) dred[tw][q] = s;
+        const double s = kb::wave_sums<2 * kStepMaxK>(da, tid & 63, q);
+        if (q >= 0) dred[tid >> 6][q] = s;
         __syncthreads();
         if (tid < 2 * nk) {
             double t = dred[0][tid];

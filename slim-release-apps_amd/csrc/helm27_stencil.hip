@@ -66,13 +66,14 @@ int stencil_chunk(const long* tiles, const int* nz, int n, int slots)
 }
 
 template <typename R>
-StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty, int pf, int ry)
+StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty, int pf, int ry, int tx)
 {
     StencilGrid g;
+    g.tx = tx == 32 ? 32 : TX;
     g.ty = (ty == 8) ? 8 : 4;
     g.pf = std::max(1, std::min(pf, 4));
     g.ry = (ry == 2 && g.ty == 8) ? 2 : 1;
-    g.tiles_x = (nx + TX - 1) / TX;
+    g.tiles_x = (nx + g.tx - 1) / g.tx;
     g.tiles_y = (ny + g.ty - 1) / g.ty;
     if (kchunk <= 0) {
         const long tiles = long(g.tiles_x) * g.tiles_y;
@@ -147,8 +148,8 @@ hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g,
     return launch_epi<R, true, true, true>(L, g, s);
 }
 
-template StencilGrid stencil_grid<double>(int, int, int, int, int, int, int);
-template StencilGrid stencil_grid<float>(int, int, int, int, int, int, int);
+template StencilGrid stencil_grid<double>(int, int, int, int, int, int, int, int);
+template StencilGrid stencil_grid<float>(int, int, int, int, int, int, int, int);
 template hipError_t launch_stencil<double>(int, StencilLaunch<double>, const StencilGrid&, hipStream_t);
 template hipError_t launch_stencil<float>(int, StencilLaunch<float>, const StencilGrid&, hipStream_t);
 

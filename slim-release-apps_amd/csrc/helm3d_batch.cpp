@@ -120,6 +120,7 @@ struct Layout {
     bool mixed = false;
     int variant = 0;
     int ty = 4, pf = 2, ry = 1;
+    bool mix = false;  // narrow and wide items in one launch
     std::vector<long> N, ld, off64, off32;
     std::vector<int> nblk, sblk, first;
     std::vector<StencilGrid> grid;
@@ -135,15 +136,29 @@ T* at(helm3d_batch* b, size_t off) { return reinterpret_cast<T*>(static_cast<cha
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
+// Work lists of unchosen shape take tiles of 32 columns by 8 rows on grids whose
+// last 64-column tile would be half empty, 64 by 4 on the others (the rule
+// looks at the item alone).  Four mixed solves of nx x 72 x 50: nx = 84 9.09 ->
+// 7.85 ms, 65 8.78 -> 7.81, 130 11.74 -> 10.19, 160 x 160 x 60 23.9 -> 21.9;
+// where the last tile is filled narrow tiles read more halo lines: 97 9.23 ->
+// 9.97, 128 9.51 -> 9.53, 240 x 240 x 60 44.3 -> 45.2.
+bool narrow_tiles(int nx) { return (((nx + 31) / 32) & 1) != 0; }
+
 // z planes per block of an item: the chosen launch shape, or the chunk for a
 // launch that holds four such items (an item's partial sums follow its chunk,
 // so the chunk must not depend on what else is in the batch).  One 48 x 48 x 40
 // grid with two right-hand sides: 4 planes 3.5 ms, 8 planes 4.3.
-int item_chunk(const helm3d_ctx* c)
+StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, bool mix)
 {
-    if (!c->grid_auto) return c->grid.kchunk;
-    const long tiles = 4L * c->grid.tiles_x * c->grid.tiles_y;
-    return stencil_chunk(&tiles, &c->n[2], 1, kSlots64);
+    const int tx = mix && narrow_tiles(c->n[0]) ? 32 : 64;
+    if (tx == 32) ty = 8;
+    int kc = c->grid.kchunk;
+    if (c->grid_auto) {
+        const StencilGrid g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], 1, ty, pf, 1, tx);
+        const long tiles = 4L * g.tiles_x * g.tiles_y;
+        kc = stencil_chunk(&tiles, &c->n[2], 1, kSlots64);
+    }
+    return stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, 1, tx);
 }
 
 template <typename R>
@@ -156,6 +171,7 @@ StencilLaunch<R> base_launch(const OpDesc<R>& op, const StencilGrid& g, void* si
     L.tiles_x = g.tiles_x;
     L.tiles_y = g.tiles_y;
     L.kchunk = g.kchunk;
+    L.narrow = g.tx == 32;
     return L;
 }
 
@@ -201,7 +217,7 @@ int helm3d_batch_item_bytes(const helm3d_ctx* c, int method, int maxinnerit, siz
     const size_t ld = size_t(slot_ld(c->N));
     const size_t slots64 = size_t(maxinnerit + 1) + (mixed ? maxinnerit : 0);
     const size_t slots32 = mixed ? S32_COUNT : 0;
-    const auto g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], item_chunk(c), c->grid.ty, c->grid.pf);
+    const StencilGrid g = item_grid(c, c->grid.ty, c->grid.pf, c->grid_auto);
     const size_t part = size_t(std::max(krylov_blocks(c->N), g.blocks)) * 2 * kMaxBasis * sizeof(double);
     *bytes = ld * (slots64 * sizeof(cpx<double>) + slots32 * sizeof(cpx<float>)) + part +
              sizeof(double) * (kSmallStride + kSc + 2 * kMaxBasis) + 4096;
@@ -242,6 +258,7 @@ int helm3d_batch_solve(helm3d_batch* B, int n, helm3d_ctx* const* ctxs, int mode
     Lo.ty = ctxs[0]->grid.ty;
     Lo.pf = ctxs[0]->grid.pf;
     Lo.ry = ctxs[0]->grid.ry;
+    Lo.mix = ctxs[0]->grid_auto;
     const int slots64 = (m + 1) + (Lo.mixed ? m : 0);
     const int slots32 = Lo.mixed ? S32_COUNT : 0;
     long tot64 = 0, tot32 = 0;
@@ -256,7 +273,7 @@ int helm3d_batch_solve(helm3d_batch* B, int n, helm3d_ctx* const* ctxs, int mode
         Lo.off32.push_back(tot32);
         tot64 += Lo.ld.back() * slots64;
         tot32 += Lo.ld.back() * slots32;
-        Lo.grid.push_back(stencil_grid<double>(c->n[0], c->n[1], c->n[2], item_chunk(c), Lo.ty, Lo.pf));
+        Lo.grid.push_back(item_grid(c, Lo.ty, Lo.pf, Lo.mix));
         Lo.nblk.push_back(krylov_blocks(c->N));
         Lo.sblk.push_back(Lo.grid.back().blocks);
         Lo.nblk_max = std::max(Lo.nblk_max, Lo.nblk.back());
@@ -415,10 +432,10 @@ int helm3d_batch_solve(helm3d_batch* B, int n, helm3d_ctx* const* ctxs, int mode
             const StencilLaunch<float>* d1 =
                 it == 0 ? d_k1first : at<StencilLaunch<float>>(B, Lo.o_k1) + size_t(par) * n;
             HIPCHK(launch_stencil_batch<float>(Lo.variant, 3, d1, d_first, n, Lo.sblk_total, d_active, Lo.ty,
-                                               Lo.pf, s, Lo.ry));
+                                               Lo.pf, s, Lo.ry, Lo.mix));
             HIPCHK(launch_breduce<float>(d_i32, d_active, n, 2, BS_RV, BT_SC, true, s));
             HIPCHK(launch_stencil_batch<float>(Lo.variant, 4, at<StencilLaunch<float>>(B, Lo.o_k2) + size_t(par) * n,
-                                               d_first, n, Lo.sblk_total, d_active, Lo.ty, Lo.pf, s, Lo.ry));
+                                               d_first, n, Lo.sblk_total, d_active, Lo.ty, Lo.pf, s, Lo.ry, Lo.mix));
             HIPCHK(launch_breduce<float>(d_i32, d_active, n, 7, BS_TS, BT_SC, true, s));
         }
         const int last = int(inner_its & 1);  // slots of the last iteration's p, r, v
@@ -524,7 +541,7 @@ int helm3d_batch_solve(helm3d_batch* B, int n, helm3d_ctx* const* ctxs, int mode
                 HIPCHK(launch_bup(d_i32, d_i64, d_active, n, nbm, S32_Z, m + 1 + (k - 1), st));
             }
             HIPCHK(launch_stencil_batch<double>(Lo.variant, 0, at<StencilLaunch<double>>(B, Lo.o_st64) + size_t(k) * n,
-                                                d_first, n, Lo.sblk_total, d_active, Lo.ty, Lo.pf, st, Lo.ry));
+                                                d_first, n, Lo.sblk_total, d_active, Lo.ty, Lo.pf, st, Lo.ry, Lo.mix));
             // classical Gram-Schmidt (FGMRES.m:100-103) on the unnormalised basis
             // streaming basis loads once the slots read per pass exceed the last-level cache
             const bool nt = double(k) * double(Lo.total_points) * sizeof(cpx<double>) > 256.0 * (1 << 20);
@@ -582,7 +599,7 @@ int helm3d_batch_solve(helm3d_batch* B, int n, helm3d_ctx* const* ctxs, int mode
         // true residual r = b - A x into slot 0 and its norm (FGMRES.m:120-124)
         CHK(set_active([&](int i) { return !S[i].done; }));
         HIPCHK(launch_stencil_batch<double>(Lo.variant, 1, at<StencilLaunch<double>>(B, Lo.o_res64), d_first, n,
-                                            Lo.sblk_total, d_active, Lo.ty, Lo.pf, st, Lo.ry));
+                                            Lo.sblk_total, d_active, Lo.ty, Lo.pf, st, Lo.ry, Lo.mix));
         HIPCHK(launch_breduce<double>(d_i64, d_active, n, 1, kNrm, BT_SMALL, true, st));
         CHK(fetch());
         bool all_below = true;

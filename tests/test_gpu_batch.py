@@ -125,6 +125,37 @@ def test_mixed_batch_uneven_grids(mode):
 
 @pytest.mark.parametrize("method", ["mixed", "plain"])
 @pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("wnc", [False, True])
+def test_batch_tile_widths(mode, method, wnc):
+    """One work list of grids on both sides of the tile-width rule (32-column
+    tiles where the last 64-column tile would be half empty): nx = 31, 33, 64,
+    65, 95 and 97, y extents that fill neither 4 nor 8 rows.  Every item
+    reaches tol with the oracle operator, and an item's solution does not
+    depend on the other items."""
+    import torch
+    from helm3d import BatchSolver, Helm3d
+    items = []
+    for nx, ny in ((31, 30), (33, 25), (64, 27), (65, 33), (95, 26), (97, 29)):
+        c, w, H = _op((nx - 12, ny - 12, 14), 6, 6.0, nx)
+        if wnc:
+            w = w * (1.0 + 0.02j)
+            H = Helm3d(c.nt, (c.h,) * 3, c.npml6, torch.from_numpy(w).to("cuda:0"))
+        items.append((c, w, H, (5, 6, 3)))
+    bs = [_rhs(c, s) for c, _, _, s in items]
+    print("tile widths mode", mode, method, wnc, flush=True)
+    v = ("forw" if mode == 1 else "adj") + ("_wnc" if wnc else "")
+    S = BatchSolver("cuda:0")
+    kw = dict(mode=mode, method=method, tol=1e-6, inner_maxit=10)
+    xs, infos = S.solve([it[2] for it in items], [torch.from_numpy(b).cuda() for b in bs], **kw)
+    for i, ((c, w, H, _), b, x, inf) in enumerate(zip(items, bs, xs, infos)):
+        r = b - O.hmvp(v, w, (c.h,) * 3, c.nt, np.array(c.npml6), x.cpu().numpy())
+        assert inf.converged and np.linalg.norm(r) < 1e-6 * np.linalg.norm(b), (i, inf)
+        if method == "mixed":
+            assert torch.equal(S.solve([H], [torch.from_numpy(b).cuda()], **kw)[0][0], x), i
+
+
+@pytest.mark.parametrize("method", ["mixed", "plain"])
+@pytest.mark.parametrize("mode", [1, 2])
 def test_batch_two_rows_per_thread(mode, method):
     """Batched solves on the 64 x 8, two-rows-per-thread launch shape (the
     fused BiCGStab passes and the FP64 work-list stencils with two output rows
