@@ -154,16 +154,16 @@ int helm3d_apply_noalloc(int variant, const int n[3], const double h[3], const i
 
 /* Stencil launch shape: z planes per block (0: automatic), column-tile rows
  * (4 or 8), planes of loads in flight (1 to 4; the batched kernels use at
- * most 2) and rows per thread (1, or 2 with 8 tile rows: 256 threads per
- * 64 x 8 tile instead of 512, so two tiles share a compute unit).  The
- * result is identical for every shape; only speed changes.  Chosen per grid
+ * most 2) and rows per thread (1: tiles of 32 columns, 64 by 4 rows in the
+ * batched kernels; or 2 with 8 tile rows: tiles of 64 columns).  The result
+ * is identical for every shape; only speed changes.  Chosen per grid
  * by the autotuner (helm3d_autotune). */
 int helm3d_set_launch(helm3d_ctx *ctx, int kchunk, int tile_rows, int prefetch, int rows_per_thread);
 int helm3d_get_launch(helm3d_ctx *ctx, int *kchunk, int *tile_rows, int *prefetch, int *rows_per_thread,
                       int *blocks);
 /* Autotuner of the stencil launch shape for this context's grid: times every
- * candidate shape (64 x 4 and 64 x 8 column tiles, the latter with one or two
- * rows per thread, prefetch {1, 2, 3, 4}, z chunks of the whole column down
+ * candidate shape (32 x 4 and 32 x 8 column tiles, and 64 x 8 with two rows
+ * per thread, prefetch {1, 2, 3, 4}, z chunks of the whole column down
  * to 8 planes, and of 4, 2 and 1 planes on grids of fewer than 128 64 x 4
  * column tiles) on the operator of `mode` (1: H, else H^H) in `precision`,
  * `reps` launches each with HIP events on the context's stream, and keeps the

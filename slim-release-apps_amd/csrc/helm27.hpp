@@ -45,7 +45,7 @@ struct StencilLaunch {
     const cpx<R>* rh;
     double* sc;
     int rho_new, rho_old, first;
-    int narrow;       // work lists: tiles_x counts tiles of 32 columns
+    int narrow;       // mixed work lists: 32 x 8 tiles
     const int* skip;  // optional (device): the launch does nothing while *skip != 0
 };
 
@@ -78,9 +78,8 @@ struct StepArgs {
     double* dpart;
 };
 
-// Launch shape: 64 x ty column tiles, z chunks of kchunk planes, pf planes of
-// loads in flight, ry rows per thread (2 only with ty = 8: 256 threads per
-// tile instead of 512).
+// Launch shape: tx x ty column tiles, z chunks of kchunk planes, pf planes of
+// loads in flight, ry rows per thread (2 only with ty = 8).
 constexpr int kSinkSlots = 65536;
 
 struct StencilGrid {
@@ -95,20 +94,25 @@ struct StencilGrid {
 //   planes = sum tiles (nz + 2 chunks), x = blocks / slots,
 // fitted to launches of chunks from 2 planes to the whole column on single
 // grids of 48 x 48 x 40 to 296 x 296 x 168 and on batches of 2 to 8 of them;
-// the chunk it picks is within 5 % of the best of the sweep on each
-// (complex128 48 x 48 x 40: 2 planes 5.7 us, 8 planes 9.8; 84^3: 8 planes 14.6,
-// 6 planes 15.8, 42 planes 34.9; complex64 240 x 240 x 140: 18 planes 47.9, 70
-// planes 58.8; six uneven grids together: 16 planes 13.7 ms, 8 planes 15.1).
+// the chunk it picks is within 8 % of the best of the sweep on each
+// (complex128 48 x 48 x 40: 2 planes 5.9 us, 7 planes 9.7; 84^3: 6 planes 12.6,
+// 9 planes 16.3, 42 planes 34.0; complex64 240 x 240 x 140: 18 planes 45.3, 70
+// planes 56.8; six uneven grids together: 16 planes 13.7 ms, 8 planes 15.1).
 // About two complex128 blocks of 256 threads fit a compute unit, four
 // complex64 ones.
 int stencil_chunk(const long* tiles, const int* nz, int n, int slots);
 constexpr int kSlots64 = 512, kSlots32 = 1024;
 
 // kchunk <= 0 picks the chunk by stencil_chunk for precision R; ty in {4, 8};
-// pf in 1..4; ry in {1, 2} (2 needs ty = 8; otherwise 1 is used).
+// pf in 1..4; ry in {1, 2} (2 needs ty = 8; otherwise 1 is used); tx = 0: tiles
+// of 32 columns, of 64 with two rows per thread.  Tiles of 32 x 8 read 1.33
+// points per output and waste no more than 31 lanes of a row, tiles of 64 x 4
+// with the same threads 1.55 and 63; and more waves lie outside the PML.
+// Against 64 x 4, complex128 forward / complex64 adjoint: 84^3 14.9 -> 12.6 /
+// 11.7 -> 9.6 us, 160 x 160 x 80 28.0 -> 23.9 / 18.9 -> 16.1, 240 x 240 x 140
+// 93.9 -> 85.9 / 54.7 -> 47.8, 280 x 280 x 140 119 -> 105 / 71.2 -> 61.5.
 template <typename R>
-StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 4, int pf = 2, int ry = 1,
-                         int tx = 64);
+StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 8, int pf = 2, int ry = 1, int tx = 0);
 
 template <typename R>
 hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g, hipStream_t s);
@@ -126,8 +130,9 @@ hipError_t launch_stencil_fused(int variant, int epi, StencilLaunch<float> L, co
 // launched with its own tiles_x/tiles_y/kchunk and the common shape (ty, pf,
 // ry: two rows per thread with ty = 8).
 // epi: 0 (y = alpha H x), 1 (+ beta b), 3, 4 (fused BiCGStab forms).
-// mix: items with narrow set have tiles of 32 columns by 8 rows (the others
-// ty x 64, ty = 4, pf = 2, ry = 1).
+// mix: items with narrow set have tiles of 32 columns by 8 rows, the others 64
+// by 4 (ty, pf, ry unused).  Otherwise all items have 64 x ty tiles, or 32 x 8
+// for ty = 8 with one row per thread.
 // active (nullable): items with active[it] == 0 do nothing.
 template <typename R>
 hipError_t launch_stencil_batch(int variant, int epi, const StencilLaunch<R>* items, const int* first, int nitems,

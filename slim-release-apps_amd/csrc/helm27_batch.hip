@@ -15,8 +15,8 @@ namespace {
 // registers.  The choice is per item and per block, so an item's bits do not
 // depend on its neighbours in the list, and the wide items of a mixed launch
 // take as long as in a launch of their own.
-template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY, bool MIX>
-__global__ __launch_bounds__(TX* TY / RY) void helm27_batch_kernel(const StencilLaunch<R>* __restrict__ items,
+template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY, bool MIX, int TXW>
+__global__ __launch_bounds__(TXW* TY / RY) void helm27_batch_kernel(const StencilLaunch<R>* __restrict__ items,
                                                               const int* __restrict__ first, int nitems,
                                                               const int* __restrict__ active)
 {
@@ -30,12 +30,12 @@ __global__ __launch_bounds__(TX* TY / RY) void helm27_batch_kernel(const Stencil
     if (active && !active[lo]) return;
     if constexpr (MIX) {
         if (items[lo].narrow) {
-            helm27_body<R, ADJ, DERIV, WNC, 2 * TY, PF, EPI, RY, TX / 2>(items[lo], bid - first[lo],
+            helm27_body<R, ADJ, DERIV, WNC, 2 * TY, PF, EPI, RY, TXW / 2>(items[lo], bid - first[lo],
                                                                          first[lo + 1] - first[lo]);
             return;
         }
     }
-    helm27_body<R, ADJ, DERIV, WNC, TY, PF, EPI, RY>(items[lo], bid - first[lo], first[lo + 1] - first[lo]);
+    helm27_body<R, ADJ, DERIV, WNC, TY, PF, EPI, RY, TXW>(items[lo], bid - first[lo], first[lo + 1] - first[lo]);
 }
 
 
@@ -45,30 +45,30 @@ hipError_t launch_b(const StencilLaunch<R>* items, const int* first, int nitems,
 {
     const dim3 grid(blocks);
     if (mix) {
-        hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 4, 2, EPI, 1, true>), grid, dim3(TX * 4), 0, s, items,
+        hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 4, 2, EPI, 1, true, 64>), grid, dim3(TX * 4), 0, s, items,
                            first, nitems, active);
         return hipGetLastError();
     }
     if (ty == 8 && ry == 2) {
         if (pf >= 2)
-            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 2, EPI, 2, false>), grid, dim3(TX * 4), 0, s, items,
+            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 2, EPI, 2, false, 64>), grid, dim3(TX * 4), 0, s, items,
                                first, nitems, active);
         else
-            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 1, EPI, 2, false>), grid, dim3(TX * 4), 0, s, items,
+            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 1, EPI, 2, false, 64>), grid, dim3(TX * 4), 0, s, items,
                                first, nitems, active);
     } else if (ty == 8) {
         if (pf >= 2)
-            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 2, EPI, 1, false>), grid, dim3(TX * 8), 0, s, items,
+            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 2, EPI, 1, false, 32>), grid, dim3(32 * 8), 0, s, items,
                                first, nitems, active);
         else
-            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 1, EPI, 1, false>), grid, dim3(TX * 8), 0, s, items,
+            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 8, 1, EPI, 1, false, 32>), grid, dim3(32 * 8), 0, s, items,
                                first, nitems, active);
     } else {
         if (pf >= 2)
-            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 4, 2, EPI, 1, false>), grid, dim3(TX * 4), 0, s, items,
+            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 4, 2, EPI, 1, false, 64>), grid, dim3(TX * 4), 0, s, items,
                                first, nitems, active);
         else
-            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 4, 1, EPI, 1, false>), grid, dim3(TX * 4), 0, s, items,
+            hipLaunchKernelGGL((helm27_batch_kernel<R, A, false, W, 4, 1, EPI, 1, false, 64>), grid, dim3(TX * 4), 0, s, items,
                                first, nitems, active);
     }
     return hipGetLastError();

@@ -10,18 +10,18 @@ namespace {
 // One shape, the one stencil_grid picks by rule: the block sums group the dots
 // by the launch's blocks, so a shape tuned per handle would give two handles of
 // one grid different inner solves.
-constexpr int kFTy = 4, kFPf = 2;
+constexpr int kFTx = 32, kFTy = 8, kFPf = 2;
 
 template <bool ADJ, bool WNC, int EPI>
-__global__ __launch_bounds__(TX* kFTy) void helm27_fused_kernel(StencilLaunch<float> L)
+__global__ __launch_bounds__(kFTx* kFTy) void helm27_fused_kernel(StencilLaunch<float> L)
 {
-    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1>(L, blockIdx.x, gridDim.x);
+    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1, kFTx>(L, blockIdx.x, gridDim.x);
 }
 
 template <bool A, bool W, int EPI>
 hipError_t launch_shape(const StencilLaunch<float>& L, const StencilGrid& g, hipStream_t s)
 {
-    hipLaunchKernelGGL((helm27_fused_kernel<A, W, EPI>), dim3(g.blocks), dim3(TX * kFTy), 0, s, L);
+    hipLaunchKernelGGL((helm27_fused_kernel<A, W, EPI>), dim3(g.blocks), dim3(kFTx * kFTy), 0, s, L);
     return hipGetLastError();
 }
 
@@ -33,7 +33,7 @@ hipError_t launch_stencil_fused(int variant, int epi, StencilLaunch<float> L, co
     L.tiles_y = g.tiles_y;
     L.kchunk = g.kchunk;
     const bool adj = variant & VAR_ADJ, wnc = variant & VAR_WNC;
-    if ((variant & VAR_DERIV) || (epi != 3 && epi != 4) || g.ty != kFTy || g.ry != 1)
+    if ((variant & VAR_DERIV) || (epi != 3 && epi != 4) || g.tx != kFTx || g.ty != kFTy || g.ry != 1)
         return hipErrorInvalidValue;
     if (epi == 3) {
         if (!adj && !wnc) return launch_shape<false, false, 3>(L, g, s);

@@ -18,13 +18,13 @@
 // The adjoint is the exact conjugate transpose: F/G take the neighbour's x/y
 // PML values and the z weights come from the neighbouring planes.
 //
-// Tiling.  A block of 64 x TY / RY threads (TY = 4 or 8 rows, RY = 1 or 2 rows
-// per thread) owns a 64 x TY column tile and marches over a z chunk.  Each plane (with a one-point x/y halo) is
-// staged once in LDS (double-buffered, one barrier per plane); the global
-// loads of the next PF planes (PF = 1..4) are in flight while a plane is
-// computed, so HBM latency overlaps the march.  Block
-// ids are remapped so consecutive tiles of the same chunk land on the same XCD
-// and share halo lines in its L2.
+// Tiling.  A block owns a column tile of 32 x 4 or 32 x 8 points, one thread
+// each, or of 64 x 8 points, two rows per thread, and marches over a z chunk.
+// Each plane (with a one-point x/y halo) is staged once in LDS (double-buffered,
+// one barrier per plane); the global loads of the next PF planes (PF = 1..4)
+// are in flight while a plane is computed, so HBM latency overlaps the march.
+// Block ids are remapped so consecutive tiles of the same chunk land on the
+// same XCD and share halo lines in its L2.
 #include <cmath>
 
 #include "helm27_body.hpp"
@@ -33,10 +33,10 @@ namespace helm3d {
 
 namespace {
 
-template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY>
-__global__ __launch_bounds__(TX* TY / RY) void helm27_kernel(StencilLaunch<R> L)
+template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY, int TXW>
+__global__ __launch_bounds__(TXW* TY / RY) void helm27_kernel(StencilLaunch<R> L)
 {
-    helm27_body<R, ADJ, DERIV, WNC, TY, PF, EPI, RY>(L, blockIdx.x, gridDim.x);
+    helm27_body<R, ADJ, DERIV, WNC, TY, PF, EPI, RY, TXW, 32>(L, blockIdx.x, gridDim.x);
 }
 
 }  // namespace
@@ -69,10 +69,10 @@ template <typename R>
 StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty, int pf, int ry, int tx)
 {
     StencilGrid g;
-    g.tx = tx == 32 ? 32 : TX;
     g.ty = (ty == 8) ? 8 : 4;
     g.pf = std::max(1, std::min(pf, 4));
     g.ry = (ry == 2 && g.ty == 8) ? 2 : 1;
+    g.tx = tx > 0 ? tx : (g.ry == 2 ? 64 : 32);
     g.tiles_x = (nx + g.tx - 1) / g.tx;
     g.tiles_y = (ny + g.ty - 1) / g.ty;
     if (kchunk <= 0) {
@@ -92,24 +92,24 @@ hipError_t launch_shape(const StencilLaunch<R>& L, const StencilGrid& g, hipStre
     const dim3 grid(g.blocks);
     if (g.ty == 8 && g.ry == 2) {
         switch (g.pf) {
-        case 1: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 1, EPI, 2>), grid, dim3(TX * 4), 0, s, L); break;
-        case 2: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 2, EPI, 2>), grid, dim3(TX * 4), 0, s, L); break;
-        case 3: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 3, EPI, 2>), grid, dim3(TX * 4), 0, s, L); break;
-        default: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 4, EPI, 2>), grid, dim3(TX * 4), 0, s, L); break;
+        case 1: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 1, EPI, 2, 64>), grid, dim3(64 * 4), 0, s, L); break;
+        case 2: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 2, EPI, 2, 64>), grid, dim3(64 * 4), 0, s, L); break;
+        case 3: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 3, EPI, 2, 64>), grid, dim3(64 * 4), 0, s, L); break;
+        default: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 4, EPI, 2, 64>), grid, dim3(64 * 4), 0, s, L); break;
         }
     } else if (g.ty == 8) {
         switch (g.pf) {
-        case 1: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 1, EPI, 1>), grid, dim3(TX * 8), 0, s, L); break;
-        case 2: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 2, EPI, 1>), grid, dim3(TX * 8), 0, s, L); break;
-        case 3: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 3, EPI, 1>), grid, dim3(TX * 8), 0, s, L); break;
-        default: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 4, EPI, 1>), grid, dim3(TX * 8), 0, s, L); break;
+        case 1: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 1, EPI, 1, 32>), grid, dim3(32 * 8), 0, s, L); break;
+        case 2: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 2, EPI, 1, 32>), grid, dim3(32 * 8), 0, s, L); break;
+        case 3: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 3, EPI, 1, 32>), grid, dim3(32 * 8), 0, s, L); break;
+        default: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 8, 4, EPI, 1, 32>), grid, dim3(32 * 8), 0, s, L); break;
         }
     } else {
         switch (g.pf) {
-        case 1: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 1, EPI, 1>), grid, dim3(TX * 4), 0, s, L); break;
-        case 2: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 2, EPI, 1>), grid, dim3(TX * 4), 0, s, L); break;
-        case 3: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 3, EPI, 1>), grid, dim3(TX * 4), 0, s, L); break;
-        default: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 4, EPI, 1>), grid, dim3(TX * 4), 0, s, L); break;
+        case 1: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 1, EPI, 1, 32>), grid, dim3(32 * 4), 0, s, L); break;
+        case 2: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 2, EPI, 1, 32>), grid, dim3(32 * 4), 0, s, L); break;
+        case 3: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 3, EPI, 1, 32>), grid, dim3(32 * 4), 0, s, L); break;
+        default: hipLaunchKernelGGL((helm27_kernel<R, A, D, W, 4, 4, EPI, 1, 32>), grid, dim3(32 * 4), 0, s, L); break;
         }
     }
     return hipGetLastError();

@@ -11,18 +11,18 @@ namespace {
 
 // One shape, the one stencil_grid picks by rule: the dots are grouped by the
 // launch's blocks, and their bits must follow the grid alone.
-constexpr int kSTy = 4, kSPf = 2;
+constexpr int kSTx = 32, kSTy = 8, kSPf = 2;
 
 template <typename R, bool ADJ, bool WNC>
-__global__ __launch_bounds__(TX* kSTy) void helm27_step_kernel(StencilLaunch<R> L, StepArgs<R> X)
+__global__ __launch_bounds__(kSTx* kSTy) void helm27_step_kernel(StencilLaunch<R> L, StepArgs<R> X)
 {
-    helm27_body<R, ADJ, false, WNC, kSTy, kSPf, 5, 1>(L, blockIdx.x, gridDim.x, &X);
+    helm27_body<R, ADJ, false, WNC, kSTy, kSPf, 5, 1, kSTx>(L, blockIdx.x, gridDim.x, &X);
 }
 
 template <typename R, bool A, bool W>
 hipError_t launch_shape(const StencilLaunch<R>& L, const StepArgs<R>& X, const StencilGrid& g, hipStream_t s)
 {
-    hipLaunchKernelGGL((helm27_step_kernel<R, A, W>), dim3(g.blocks), dim3(TX * kSTy), 0, s, L, X);
+    hipLaunchKernelGGL((helm27_step_kernel<R, A, W>), dim3(g.blocks), dim3(kSTx * kSTy), 0, s, L, X);
     return hipGetLastError();
 }
 
@@ -35,7 +35,7 @@ hipError_t launch_stencil_step(int variant, StencilLaunch<R> L, const StepArgs<R
     L.tiles_x = g.tiles_x;
     L.tiles_y = g.tiles_y;
     L.kchunk = g.kchunk;
-    if ((variant & VAR_DERIV) || X.k < 1 || X.k > kStepMaxK || g.ty != kSTy || g.ry != 1)
+    if ((variant & VAR_DERIV) || X.k < 1 || X.k > kStepMaxK || g.tx != kSTx || g.ty != kSTy || g.ry != 1)
         return hipErrorInvalidValue;
     const bool adj = variant & VAR_ADJ, wnc = variant & VAR_WNC;
     if (!adj && !wnc) return launch_shape<R, false, false>(L, X, g, s);

@@ -148,17 +148,21 @@ bool narrow_tiles(int nx) { return (((nx + 31) / 32) & 1) != 0; }
 // launch that holds four such items (an item's partial sums follow its chunk,
 // so the chunk must not depend on what else is in the batch).  One 48 x 48 x 40
 // grid with two right-hand sides: 4 planes 3.5 ms, 8 planes 4.3.
-StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, bool mix)
+StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, int ry, bool mix)
 {
-    const int tx = mix && narrow_tiles(c->n[0]) ? 32 : 64;
-    if (tx == 32) ty = 8;
+    if (mix) {
+        ty = narrow_tiles(c->n[0]) ? 8 : 4;
+        pf = 2;
+        ry = 1;
+    }
+    const int tx = ty == 8 && ry == 1 ? 32 : 64;
     int kc = c->grid.kchunk;
     if (c->grid_auto) {
-        const StencilGrid g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], 1, ty, pf, 1, tx);
+        const StencilGrid g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], 1, ty, pf, ry, tx);
         const long tiles = 4L * g.tiles_x * g.tiles_y;
         kc = stencil_chunk(&tiles, &c->n[2], 1, kSlots64);
     }
-    return stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, 1, tx);
+    return stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, ry, tx);
 }
 
 template <typename R>
@@ -217,7 +221,7 @@ int helm3d_batch_item_bytes(const helm3d_ctx* c, int method, int maxinnerit, siz
     const size_t ld = size_t(slot_ld(c->N));
     const size_t slots64 = size_t(maxinnerit + 1) + (mixed ? maxinnerit : 0);
     const size_t slots32 = mixed ? S32_COUNT : 0;
-    const StencilGrid g = item_grid(c, c->grid.ty, c->grid.pf, c->grid_auto);
+    const StencilGrid g = item_grid(c, c->grid.ty, c->grid.pf, c->grid.ry, c->grid_auto);
     const size_t part = size_t(std::max(krylov_blocks(c->N), g.blocks)) * 2 * kMaxBasis * sizeof(double);
     *bytes = ld * (slots64 * sizeof(cpx<double>) + slots32 * sizeof(cpx<float>)) + part +
              sizeof(double) * (kSmallStride + kSc + 2 * kMaxBasis) + 4096;
@@ -273,7 +277,7 @@ int helm3d_batch_solve(helm3d_batch* B, int n, helm3d_ctx* const* ctxs, int mode
         Lo.off32.push_back(tot32);
         tot64 += Lo.ld.back() * slots64;
         tot32 += Lo.ld.back() * slots32;
-        Lo.grid.push_back(item_grid(c, Lo.ty, Lo.pf, Lo.mix));
+        Lo.grid.push_back(item_grid(c, Lo.ty, Lo.pf, Lo.ry, Lo.mix));
         Lo.nblk.push_back(krylov_blocks(c->N));
         Lo.sblk.push_back(Lo.grid.back().blocks);
         Lo.nblk_max = std::max(Lo.nblk_max, Lo.nblk.back());

@@ -970,8 +970,8 @@ int helm3d_autotune(helm3d_ctx* c, int mode, int precision, int reps, int* kchun
             if (kc < c->n[2] && std::find(chunks.begin(), chunks.end(), kc) == chunks.end()) chunks.push_back(kc);
         }
     }
-    // (tile rows, rows per thread): 64 x 4 and 64 x 8 tiles, the latter also
-    // with two rows per thread
+    // (tile rows, rows per thread): tiles of 32 x 4, 32 x 8 and, with two rows
+    // per thread, 64 x 8
     const int shapes[3][2] = {{4, 1}, {8, 1}, {8, 2}};
     for (const auto& sh : shapes) {
         const int ty = sh[0], ry = sh[1];

@@ -47,9 +47,8 @@ class BatchSolver:
                  inner_maxit: int = 25, tile_rows=(4, 8), prefetch=(1, 2), divisors=(1, 2, 3, 4),
                  rows_per_thread=(1, 2)) -> dict:
         """Choose the stencil launch shape of a batch by timing a short batched
-        solve (one restart cycle of two outer steps) for every candidate: 64 x
-        tile_rows column tiles (64 x 8 with one or two rows per thread),
-        prefetch depth, and z chunks of nz/divisor for every operator.  The
+        solve (one restart cycle of two outer steps) for every candidate: 64 x 4
+        and 32 x 8 column tiles, 64 x 8 with two rows per thread, prefetch depth, and z chunks of nz/divisor for every operator.  The
         fastest shape is left set on the operators; later solves converge to
         the same tolerance whatever the shape (the fused BiCGStab partial sums
         follow the shape, so iteration counts can move by a few)."""

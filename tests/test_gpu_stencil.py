@@ -156,6 +156,35 @@ def test_degenerate_grids(case):
             assert torch.equal(a, b), (shape, k)
 
 
+EDGES = [(31, 7, 3), (32, 8, 2), (33, 9, 5), (63, 5, 4), (64, 4, 1), (65, 17, 6), (97, 16, 9)]
+
+
+@pytest.mark.parametrize("n", EDGES)
+def test_tile_edges(n):
+    """Grids that end on, before and behind a tile edge in x (32 and 64
+    columns) and y (4 and 8 rows), PML of one and two points so that groups of
+    32 columns lie on both sides of the interior test: complex128 (rounding of
+    27 products, bar 1e-12) and complex64 (bar 2e-6) against the oracle, and
+    bit-identical across the tile shapes."""
+    import torch
+    from helm3d import Helm3d
+    npml, h = np.array([[1, 1, 0], [2, 1, 0]]), (10.0, 11.0, 12.0)
+    dev = torch.device("cuda:0")
+    for wnc in (False, True):
+        wn, x = _inputs(n, 900 + n[0], wnc)
+        H = Helm3d(n, h, npml, torch.from_numpy(wn).to(dev))
+        xt = torch.from_numpy(x).to(dev)
+        ref = None
+        for shape in (None, (1, 4, 1, 1), (2, 4, 3, 1), (0, 8, 4, 1), (0, 8, 1, 2)):
+            if shape:
+                H.set_launch(*shape)
+            got = [H.apply(v, adjoint=a) for v in (xt, xt.to(torch.complex64)) for a in (False, True)]
+            ref = ref or got
+            assert all(torch.equal(a, b) for a, b in zip(got, ref)), shape
+        for y, v, bar in zip(ref, ("forw", "adj") * 2, (1e-12, 1e-12, 2e-6, 2e-6)):
+            assert relerr(y.cpu().numpy(), O.hmvp(v + ("_wnc" if wnc else ""), wn, h, n, npml, x)) <= bar, (v, wnc)
+
+
 SHAPES = [(0, 4, 1, 1), (35, 4, 2, 1), (70, 8, 1, 1), (17, 8, 2, 1), (23, 4, 3, 1), (9, 8, 4, 1), (70, 4, 4, 1),
           (0, 8, 1, 2), (70, 8, 2, 2), (17, 8, 3, 2), (9, 8, 4, 2),
           (1, 4, 2, 1), (1, 8, 4, 1), (2, 4, 3, 1), (2, 8, 2, 2), (4, 4, 1, 1), (1, 8, 1, 2)]
