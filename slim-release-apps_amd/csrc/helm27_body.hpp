@@ -115,7 +115,8 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     constexpr int NS = HX * HY;          // halo tile slots
     constexpr int NSL = (NS + NT - 1) / NT;  // load slots per thread
     static_assert(PF >= 1 && PF <= 4, "prefetch depth 1 to 4");
-    if (L.skip && *L.skip) return;  // uniform over the launch
+    // uniform over the launch; EPI 5 looks after its first loads are on the way
+    if (EPI != 5 && L.skip && *L.skip) return;
     const OpDesc<R>& op = L.op;
     __shared__ cpx<R> su[2][HY][HX];            // input vector plane (+halo)
     // forward mass operand: wn .* x (WNC, DERIV) or the real wn itself, the
@@ -291,31 +292,6 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     for (int r = 0; r < RY; ++r) Xlast[r] = Rlast[r] = Dlast[r] = zero<R>();
     // output scale: alpha, or alpha / sqrt(*anrm) with the norm held on the device
     R alpha = (EPI <= 1 && L.anrm) ? R(double(L.alpha) / sqrt(*L.anrm)) : L.alpha;
-    if (EPI == 5 && X->npart) {
-        // every wave adds the partials of ||x||^2 in the same order
-        double s = 0.0;
-        for (int q = tid & 63; q < X->npn; q += 64) s += X->npart[q];
-        s = kb::wave_sum(s);
-        bool stop = false;
-        if (X->start) {
-            const double b = sqrt(s);
-            stop = X->start == 1 ? b == 0.0 : b / X->st->normr0 < X->tol;
-            if (lin == 0 && tid == 0) {
-                if (X->start == 1) {
-                    X->st->normr0 = b;
-                    X->st->hlast = 1.0;
-                }
-                X->st->beta = b;
-                X->st->skip = stop ? 1 : 0;
-            }
-        }
-        if (lin == 0 && tid == 0) {
-            *X->nrm = s;
-            if (X->row) *X->row = s;
-        }
-        if (stop) return;  // the same decision in every block
-        alpha = R(double(L.alpha) / sqrt(s));
-    }
 
     // One register set: halo slots of plane q and the own-point operands of
     // plane q-1 (the plane output when q is staged).  Every load is issued
@@ -670,6 +646,34 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
         if (p > 0) __builtin_amdgcn_sched_barrier(0);
         fetch(k0 - 1 + p, S[p]);
     }
+    if constexpr (EPI == 5) {
+        if (L.skip && *L.skip) return;
+    }
+    if (EPI == 5 && X->npart) {
+        // every wave adds the partials of ||x||^2 in the same order
+        double s = 0.0;
+        for (int q = tid & 63; q < X->npn; q += 64) s += X->npart[q];
+        s = kb::wave_sum(s);
+        bool stop = false;
+        if (X->start) {
+            const double b = sqrt(s);
+            stop = X->start == 1 ? b == 0.0 : b / X->st->normr0 < X->tol;
+            if (lin == 0 && tid == 0) {
+                if (X->start == 1) {
+                    X->st->normr0 = b;
+                    X->st->hlast = 1.0;
+                }
+                X->st->beta = b;
+                X->st->skip = stop ? 1 : 0;
+            }
+        }
+        if (lin == 0 && tid == 0) {
+            *X->nrm = s;
+            if (X->row) *X->row = s;
+        }
+        if (stop) return;  // the same decision in every block
+        alpha = R(double(L.alpha) / sqrt(s));
+    }
     const int ntrips = (k1 - k0 + 2 + PF - 1) / PF;
     for (int trp = 0; trp < ntrips; ++trp) {
         const int q = k0 - 1 + trp * PF;
@@ -684,18 +688,28 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
 #pragma unroll
         for (int q = 0; q < 2 * kStepMaxK; ++q) da[q] = 0.0;
         const int nk = X->k;
-        for (int kk = k0; kk < k1; ++kk) {
+        // (two planes at a time: the loads of both are in flight together)
+        auto dots_at = [&](cpx<R> w, const cpx<R>(&v)[kStepMaxK]) {
 #pragma unroll
-            for (int r = 0; r < RY; ++r) {
-                if (!active[r]) continue;
-                const long t = long(kk) * plane + offc[r];
-                const cpx<R> w = L.y[t];
-                cpx<R> v[kStepMaxK];
+            for (int c = 0; c < kStepMaxK; ++c)
+                if (c < nk) kb::acc_dot(da[2 * c], da[2 * c + 1], v[c], w);
+        };
 #pragma unroll
-                for (int c = 0; c < kStepMaxK; ++c) v[c] = c < nk ? X->V[c * X->ldv + t] : zero<R>();
+        for (int r = 0; r < RY; ++r) {
+            if (!active[r]) continue;
+            for (int kk = k0; kk < k1; kk += 2) {
+                const long t0 = long(kk) * plane + offc[r], t1 = long(min(kk + 1, k1 - 1)) * plane + offc[r];
+                const cpx<R> w0 = L.y[t0];
+                cpx<R> w1 = L.y[t1];
+                cpx<R> v0[kStepMaxK], v1[kStepMaxK];
 #pragma unroll
-                for (int c = 0; c < kStepMaxK; ++c)
-                    if (c < nk) kb::acc_dot(da[2 * c], da[2 * c + 1], v[c], w);
+                for (int c = 0; c < kStepMaxK; ++c) {
+                    v0[c] = c < nk ? X->V[c * X->ldv + t0] : zero<R>();
+                    v1[c] = c < nk ? X->V[c * X->ldv + t1] : zero<R>();
+                }
+                if (kk + 1 >= k1) w1 = zero<R>();
+                dots_at(w0, v0);
+                dots_at(w1, v1);
             }
         }
         __shared__ double dred[NT / 64][2 * kStepMaxK];
@@ -714,12 +728,9 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     // part[q*G + lin] for q < NV
     if (L.norm_part) {
         __shared__ double red[NV][NT / 64];
-#pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            double v = acc[q];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            if ((tid & 63) == 0) red[q][tid >> 6] = v;
-        }
+        int q;
+        const double v = kb::wave_sums<NV>(acc, tid & 63, q);
+        if (q >= 0) red[q][tid >> 6] = v;
         __syncthreads();
         if (tid < NV) {
             double s = 0;

@@ -16,34 +16,6 @@ namespace kb {
 
 constexpr int KB = 256;  // threads per block
 
-__device__ inline double wave_sum(double v)
-{
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// Block-wide sums of NV values per thread; results valid in thread 0.
-template <int NV>
-__device__ inline void block_sum(double (&v)[NV], double* red /* [KB/64][NV] */)
-{
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; ++q) v[q] = wave_sum(v[q]);
-    if (lane == 0) {
-#pragma unroll
-        for (int q = 0; q < NV; ++q) red[wid * NV + q] = v[q];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            double s = red[q];
-            for (int w = 1; w < KB / 64; ++w) s += red[w * NV + q];
-            v[q] = s;
-        }
-    }
-}
-
 // Sums of NV values per lane over a wave, one or two lanes ending up with each:
 // at every step a lane hands half of its values to its partner and keeps the
 // other half, so NV + NV/2 + ... values cross lanes instead of 6 NV.  The
@@ -124,6 +96,36 @@ __device__ inline double wave_sums(double (&v)[NV], int lane, int& q)
     const double s = wave_sums_step<32, NV>(v, lane, base, end);
     q = base < end ? base : -1;
     return s;
+}
+
+// Sum of one value per lane, in every lane.
+__device__ inline double wave_sum(double v)
+{
+    double a[1] = {v};
+    int base = 0, end = 1;
+    return wave_sums_step<32, 1>(a, int(threadIdx.x & 63), base, end);
+}
+
+// Block-wide sums of NV values per thread; results valid in thread 0.
+template <int NV>
+__device__ inline void block_sum(double (&v)[NV], double* red /* [KB/64][NV] */)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) v[q] = wave_sum(v[q]);
+    if (lane == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) red[wid * NV + q] = v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            double s = red[q];
+            for (int w = 1; w < KB / 64; ++w) s += red[w * NV + q];
+            v[q] = s;
+        }
+    }
 }
 
 // Block-wide sums of NV values per thread into part[q * G + b], q < NV: waves

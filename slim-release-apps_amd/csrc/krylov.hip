@@ -55,13 +55,19 @@ __global__ __launch_bounds__(KB) void update_kernel(const cpx<R>* __restrict__ V
     if (skip && *skip) return;
     __shared__ double dsum[2 * K];
     if (dpart) {
+        // a wave's columns together: their loads and exchanges overlap
+        constexpr int NQ = (2 * K + KB / 64 - 1) / (KB / 64);
         const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-        for (int q = wid; q < 2 * K; q += KB / 64) {
-            double s = 0.0;
-            for (int b = lane; b < dnblk; b += 64) s += dpart[long(q) * dnblk + b];
-            s = kb::wave_sum(s);
-            if (lane == 0) dsum[q] = s;
+        double s[NQ];
+#pragma unroll
+        for (int i = 0; i < NQ; ++i) s[i] = 0.0;
+        for (int b = lane; b < dnblk; b += 64) {
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) s[i] += dpart[long(min(wid * NQ + i, 2 * K - 1)) * dnblk + b];
         }
+        int i;
+        const double v = kb::wave_sums<NQ>(s, lane, i);
+        if (i >= 0 && wid * NQ + i < 2 * K) dsum[wid * NQ + i] = v;
         __syncthreads();
         if (blockIdx.x == 0 && threadIdx.x < 2 * K) hrow[threadIdx.x] = dsum[threadIdx.x];
     }
