@@ -647,7 +647,11 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
         fetch(k0 - 1 + p, S[p]);
     }
     if constexpr (EPI == 5) {
-        if (L.skip && *L.skip) return;
+        if (L.skip && *L.skip) {
+            // a stopped solve: the rest of the cycle looks at skip
+            if (X->start == 2 && lin == 0 && tid == 0) X->st->skip = 1;
+            return;
+        }
     }
     if (EPI == 5 && X->npart) {
         // every wave adds the partials of ||x||^2 in the same order

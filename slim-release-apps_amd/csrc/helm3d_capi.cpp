@@ -234,7 +234,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
     // Device-driven solves of short vectors: two launches per Arnoldi step.
     // The step launch (matvec and dots) sums the partials that the update pass
     // (or the start) left of its input's norm, the update pass the dots; the
-    // first step of a cycle takes the stop decisions, the least squares the
+    // first step of a cycle takes the stop decisions, the end of the cycle the
     // norm of the last slot.  Partials: norms at the front, dots behind them.
     // Launched one by one: as captured graphs the short cycles took 3 to 5 %
     // longer, alone and with four hierarchies at once.
@@ -250,7 +250,7 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
                 L.y = slot(j);
                 L.alpha = R(1);
                 L.sink = static_cast<cpx<R>*>(c->sink);
-                L.skip = start == 1 && j == 1 ? nullptr : &st->skip;
+                L.skip = j > 1 ? &st->skip : (start == 1 ? nullptr : &st->stop);
                 StepArgs<R> X{};
                 X.npart = c->part;
                 X.npn = j == 1 ? npn : nblk;
@@ -268,17 +268,17 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
                       launch_update<R>(V, ld, j, nullptr, CoefPack{}, slot(j), N, c->part, nblk, s, c->nrm, dpart,
                                        G.blocks, c->gs + size_t(j) * kGsRow, &st->skip));
             }
-            HIPCHK(launch_gmres_lsq(c->gs, kGsRow, m, tol, st, s, c->part, nblk));
             return HELM3D_OK;
         };
         for (long cyc = 0; (1 + cyc * long(m)) / m < maxit; ++cyc) {
             const bool resid = cyc > 0 || use_x0;
-            if (resid) CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, cyc > 0 ? skip : nullptr, &G));
+            if (resid)
+                CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, cyc > 0 ? &st->stop : nullptr, &G));
             else HIPCHK(launch_start<R>(b, slot(0), x, N, c->part, nblk, c->stream));
             const int start = cyc > 0 ? 2 : 1, npn = resid ? G.blocks : nblk;
             CHK(steps(c->stream, start, npn));
             TIMED(HELM3D_PROF_COMBINE,
-                  launch_combine_dev<R>(V, ld, m, st->coef, &st->kept, x, N, nblk_u, c->stream, nullptr));
+                  launch_cycle_end<R>(V, ld, m, c->gs, kGsRow, tol, st, c->part, nblk, x, N, c->stream));
         }
         res->iters = -1;
         res->cycles = -1;

@@ -174,22 +174,20 @@ __global__ void gmres_restart_kernel(const double* __restrict__ nrm, double tol,
 // side g), so the quasi-residual of step k is |g_k| / ||r0|| -- the residual
 // of the k-step least squares -- after O(k) work.  Steps after the first one
 // at or below tol are dropped (the host loop would not have run them); coef
-// receives a_q = y_q sig_q for the kept steps, zeros after.  One thread.
+// receives a_q = y_q sig_q for the kept steps, zeros after (q < MB).  One thread.
 // Cycles of at most MB steps; MB = kMaxBasis keeps T, g and the rotations in
 // LDS, smaller MB in registers (every index fixed once the loops unroll).
 template <int MB>
 __device__ __forceinline__ void gmres_lsq_body(const double* __restrict__ rows, int ldr, int m, double tol,
-                                               GmresDevState* st, Cx* T, Cx* cs, Cx* sn, Cx* g, Cx* y,
-                                               double* sig)
+                                               double beta, double normr0, Cx* T, Cx* cs, Cx* sn, Cx* g, Cx* y,
+                                               double* sig, double* __restrict__ coef, int& kept, double& hlast)
 {
     constexpr int ld = MB + 1;
     // unrolled (register arrays) for short cycles, rolled for the LDS form
     constexpr int kU = MB <= 5 ? MB + 1 : 1;
-    const double normr0 = st->normr0;
-    sig[0] = 1.0 / st->beta;
-    g[0] = Cx{st->beta, 0.0};
-    int kept = m;
-    double hlast = st->hlast;
+    sig[0] = 1.0 / beta;
+    g[0] = Cx{beta, 0.0};
+    kept = m;
 #pragma unroll kU
     for (int k = 1; k <= MB; ++k) {
         if (k > m) break;
@@ -236,42 +234,118 @@ __device__ __forceinline__ void gmres_lsq_body(const double* __restrict__ rows, 
         }
     }
 #pragma unroll kU
-    for (int q = 0; q < kMaxBasis; ++q) {
-        const Cx a = (q < MB && q < kept) ? cx_scale(y[q < MB ? q : 0], sig[q < MB ? q : 0]) : Cx{0.0, 0.0};
-        st->coef[2 * q] = a.re;
-        st->coef[2 * q + 1] = a.im;
+    for (int q = 0; q < MB; ++q) {
+        const Cx a = q < kept ? cx_scale(y[q], sig[q]) : Cx{0.0, 0.0};
+        coef[2 * q] = a.re;
+        coef[2 * q + 1] = a.im;
+    }
+}
+
+template <int MB>
+__global__ __launch_bounds__(64) void gmres_lsq_kernel(const double* __restrict__ rows, int ldr, int m, double tol,
+                                                       GmresDevState* st)
+{
+    if (st->skip) return;
+    if (threadIdx.x != 0) return;
+    int kept;
+    double hlast;
+    if constexpr (MB == kMaxBasis) {
+        __shared__ Cx T[(MB + 1) * MB];
+        __shared__ Cx cs[MB], sn[MB], g[MB + 1], y[MB];
+        __shared__ double sig[MB + 1];
+        gmres_lsq_body<MB>(rows, ldr, m, tol, st->beta, st->normr0, T, cs, sn, g, y, sig, st->coef, kept, hlast);
+    } else {
+        Cx T[(MB + 1) * MB], cs[MB], sn[MB], g[MB + 1], y[MB];
+        double sig[MB + 1];
+        gmres_lsq_body<MB>(rows, ldr, m, tol, st->beta, st->normr0, T, cs, sn, g, y, sig, st->coef, kept, hlast);
     }
     st->hlast = hlast;
     st->kept = kept;
     if (hlast <= tol) st->stop = 1;
 }
 
-template <int MB>
-__global__ __launch_bounds__(64) void gmres_lsq_kernel(double* rows, int ldr, int m, double tol, GmresDevState* st,
-                                                       const double* npart, int npn)
+// End of a cycle of K steps on a short vector (launch_stencil_step): every block
+// runs the least squares itself and adds its points of x += V y, so the cycle
+// has no one-block launch.  rows[1..K] hold the steps' dots and norms but for
+// ||slot(K)||^2, summed here from the update pass's partials.  Reads skip, beta
+// and normr0, which no block of the launch writes; the decision for the next
+// cycle goes to stop.  The rows and the block's first points are loaded ahead
+// of the one-thread least squares, which takes most of the time (8211 points,
+// K = 5: 8.2 us for the one-block launch and 3.7 us for the update before).
+template <typename R, int K>
+__global__ __launch_bounds__(KB) void cycle_end_kernel(const cpx<R>* __restrict__ V, long ldv,
+                                                       const double* __restrict__ rows, int ldr, double tol,
+                                                       GmresDevState* st, const double* __restrict__ npart, int npn,
+                                                       cpx<R>* __restrict__ x, long n)
 {
-    if (st->skip) {
-        if (npart && threadIdx.x == 0) st->kept = 0;
+    constexpr int W = 2 * K + 1;
+    __shared__ double srow[(K + 1) * W], coef[2 * K];
+    __shared__ int skept;
+    const int tid = threadIdx.x;
+    long lo, hi;
+    kb::range_even(n, blockIdx.x, gridDim.x, lo, hi);
+    long t = lo + tid;
+    cpx<R> v[K], xt = cpx<R>{R(0), R(0)};
+    auto load = [&]() {
+#pragma unroll
+        for (int c = 0; c < K; ++c) v[c] = t < hi ? V[c * ldv + t] : cpx<R>{R(0), R(0)};
+        if (t < hi) xt = x[t];
+    };
+    load();
+    for (int q = tid; q < K * W; q += KB) {
+        const int k = 1 + q / W, e = q % W;
+        if (e <= 2 * k && !(k == K && e == 2 * K)) srow[k * W + e] = rows[long(k) * ldr + e];
+    }
+    if (tid < 64) {
+        double s = 0.0;
+        for (int q = tid; q < npn; q += 64) s += npart[q];
+        s = kb::wave_sum(s);
+        if (tid == 0) srow[K * W + 2 * K] = s;
+    }
+    const int skip = st->skip;
+    const double beta = st->beta, normr0 = st->normr0;
+    __syncthreads();
+    if (skip) {
+        if (blockIdx.x == 0 && tid == 0) st->stop = 1;
         return;
     }
-    if (npart) {
-        double s = 0.0;
-        for (int q = threadIdx.x; q < npn; q += 64) s += npart[q];
-        s = kb::wave_sum(s);
-        if (threadIdx.x == 0) rows[long(m) * ldr + 2 * m] = s;
+    if constexpr (K > 5) {
+        __shared__ Cx T[(K + 1) * K];
+        __shared__ Cx cs[K], sn[K], g[K + 1], y[K];
+        __shared__ double sig[K + 1];
+        if (tid == 0) {
+            int kept;
+            double hlast;
+            gmres_lsq_body<K>(srow, W, K, tol, beta, normr0, T, cs, sn, g, y, sig, coef, kept, hlast);
+            skept = kept;
+            if (blockIdx.x == 0) st->stop = hlast <= tol ? 1 : 0;
+        }
+    } else if (tid == 0) {
+        Cx T[(K + 1) * K], cs[K], sn[K], g[K + 1], y[K];
+        double sig[K + 1];
+        int kept;
+        double hlast;
+        gmres_lsq_body<K>(srow, W, K, tol, beta, normr0, T, cs, sn, g, y, sig, coef, kept, hlast);
+        skept = kept;
+        if (blockIdx.x == 0) st->stop = hlast <= tol ? 1 : 0;
     }
-    if (threadIdx.x != 0) return;
-    if constexpr (MB == kMaxBasis) {
-        __shared__ Cx T[(MB + 1) * MB];
-        __shared__ Cx cs[MB], sn[MB], g[MB + 1], y[MB];
-        __shared__ double sig[MB + 1];
-        gmres_lsq_body<MB>(rows, ldr, m, tol, st, T, cs, sn, g, y, sig);
-    } else {
-        Cx T[(MB + 1) * MB], cs[MB], sn[MB], g[MB + 1], y[MB];
-        double sig[MB + 1];
-        gmres_lsq_body<MB>(rows, ldr, m, tol, st, T, cs, sn, g, y, sig);
+    __syncthreads();
+    const int kk = skept;
+    while (t < hi) {
+        double re = xt.re, im = xt.im;
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            if (c < kk) {
+                re = fma(coef[2 * c], double(v[c].re), re);
+                re = fma(-coef[2 * c + 1], double(v[c].im), re);
+                im = fma(coef[2 * c], double(v[c].im), im);
+                im = fma(coef[2 * c + 1], double(v[c].re), im);
+            }
+        }
+        x[t] = cpx<R>{R(re), R(im)};
+        t += KB;
+        load();
     }
-    if (npart && st->hlast <= tol) st->skip = 1;
 }
 
 // out[q] = sum_b part[q*nblk + b] in block order; one block per column q
@@ -558,17 +632,28 @@ hipError_t launch_gmres_restart(const double* nrm, double tol, GmresDevState* st
     hipLaunchKernelGGL(gmres_restart_kernel, dim3(1), dim3(1), 0, s, nrm, tol, st);
     return hipGetLastError();
 }
-hipError_t launch_gmres_lsq(double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s,
-                            const double* npart, int npn)
+hipError_t launch_gmres_lsq(const double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s)
 {
     if (m < 1 || m >= kMaxBasis) return hipErrorInvalidValue;
-    if (m <= 2)
-        hipLaunchKernelGGL(gmres_lsq_kernel<2>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st, npart, npn);
-    else if (m <= 5)
-        hipLaunchKernelGGL(gmres_lsq_kernel<5>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st, npart, npn);
-    else
-        hipLaunchKernelGGL(gmres_lsq_kernel<kMaxBasis>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st, npart, npn);
+    if (m <= 2) hipLaunchKernelGGL(gmres_lsq_kernel<2>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st);
+    else if (m <= 5) hipLaunchKernelGGL(gmres_lsq_kernel<5>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st);
+    else hipLaunchKernelGGL(gmres_lsq_kernel<kMaxBasis>, dim3(1), dim3(64), 0, s, rows, ldr, m, tol, st);
     return hipGetLastError();
+}
+
+template <typename R>
+hipError_t launch_cycle_end(const cpx<R>* V, long ldv, int m, const double* rows, int ldr, double tol,
+                            GmresDevState* st, const double* npart, int npn, cpx<R>* x, long n, hipStream_t s)
+{
+    if (m < 1 || m > kStepMaxK) return hipErrorInvalidValue;
+    const int nblk = krylov_blocks(n);
+    return dispatch_k<1>(m, [&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        if constexpr (K <= kStepMaxK)
+            hipLaunchKernelGGL((cycle_end_kernel<R, K>), dim3(nblk), dim3(KB), 0, s, V, ldv, rows, ldr, tol, st, npart,
+                               npn, x, n);
+        return hipGetLastError();
+    });
 }
 
 template <typename R>
@@ -665,6 +750,8 @@ hipError_t launch_start(const cpx<R>* b, cpx<R>* w, cpx<R>* x, long n, double* p
                                          int, double*, const int*);                                         \
     template hipError_t launch_combine_dev<R>(const cpx<R>*, long, int, const double*, const int*, cpx<R>*, \
                                               long, int, hipStream_t, const int*);                          \
+    template hipError_t launch_cycle_end<R>(const cpx<R>*, long, int, const double*, int, double,           \
+                                            GmresDevState*, const double*, int, cpx<R>*, long, hipStream_t); \
     template hipError_t launch_combine<R>(const cpx<R>*, long, int, const CoefPack&, cpx<R>*, long, int,    \
                                           hipStream_t);                                                     \
     template hipError_t launch_norm2<R>(const cpx<R>*, long, double*, int, hipStream_t);

@@ -73,11 +73,14 @@ hipError_t launch_combine_dev(const cpx<R>* V, long ldv, int k, const double* a,
 hipError_t launch_gmres_start(const double* nrm, GmresDevState* st, hipStream_t s);
 hipError_t launch_gmres_gate(GmresDevState* st, hipStream_t s);
 hipError_t launch_gmres_restart(const double* nrm, double tol, GmresDevState* st, hipStream_t s);
-// npart (optional): ||w_m||^2 is summed from these npn partials first, and a
-// cycle that the state skips leaves kept = 0, so that the combine needs no flag
-// and a stop skips the following cycles' steps.
-hipError_t launch_gmres_lsq(double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s,
-                            const double* npart = nullptr, int npn = 0);
+hipError_t launch_gmres_lsq(const double* rows, int ldr, int m, double tol, GmresDevState* st, hipStream_t s);
+// End of a cycle of m steps on a short vector (m <= 8): least squares and
+// x += V y in one launch of krylov_blocks(n) blocks; ||slot(m)||^2 is summed
+// from npart (npn partials).  A cycle with st->skip set leaves x as it is;
+// st->stop tells the next cycle.
+template <typename R>
+hipError_t launch_cycle_end(const cpx<R>* V, long ldv, int m, const double* rows, int ldr, double tol,
+                            GmresDevState* st, const double* npart, int npn, cpx<R>* x, long n, hipStream_t s);
 hipError_t launch_interleave(const double* re, const double* im, cpx<double>* z, long n, hipStream_t s);
 hipError_t launch_deinterleave(const cpx<double>* z, double* re, double* im, long n, hipStream_t s);
 // b = a, c = float(a)
