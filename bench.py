@@ -472,9 +472,10 @@ def kacz_leg(sweeps=5):
     """The Kaczmarz path (Helm3dkaczswp_mex.c, CGMN.m, CRMN.m): double sweeps
     of the 240x240x140 benchmark model timed with events (forward and adjoint
     rows), and CGMN and CRMN solves of the C1 problem (64^3 + 10-pt PML, 5 Hz)
-    to 1e-6.  Algorithmic bytes of a double sweep: each of the 54 colour
-    launches reads and writes x at every point and reads wn (40 B/pt), and
-    each row reads b once per direction (2 x 16 B/pt): 2192 B/pt."""
+    to 1e-6.  Algorithmic bytes of a double sweep: the 18 row classes run
+    in 17 launches (the last class of the way up is the first of the way
+    down), each of which reads and writes x at every point and reads wn (40
+    B/pt), and each row reads b once per direction (2 x 16 B/pt): 712 B/pt."""
     import numpy as np
     import torch
     from helm3d import Helm3d
@@ -486,7 +487,7 @@ def kacz_leg(sweeps=5):
     rng = np.random.default_rng(3)
     x = torch.from_numpy(rng.standard_normal(H.N) + 1j * rng.standard_normal(H.N)).to(dev)
     b = torch.from_numpy(rng.standard_normal(H.N) + 1j * rng.standard_normal(H.N)).to(dev)
-    alg = 2192.0 * H.N
+    alg = 712.0 * H.N
     out = {"workload": "double Kaczmarz sweeps (27-colour order, omega 1.5) on the 240x240x140 benchmark model; "
                        "CGMN and CRMN solves of C1 (64^3 + 10-pt PML, 5 Hz, one impulse) to 1e-6",
            "alg_bytes_per_double_sweep": alg}

@@ -38,7 +38,7 @@ struct MgLevel {
 struct AxisTab {
     std::vector<int> I, rp, fi, pfi;
     std::vector<double> wa, wb, fw, pfw;
-    int pw = 0;
+    int pw = 0, run = 0;
 };
 
 AxisTab axis_tab(int nf, int nc)
@@ -90,6 +90,21 @@ AxisTab axis_tab(int nf, int nc)
             t.pfi[size_t(c) * t.pw + e] = real ? t.fi[q] : (t.rp[c] < t.rp[c + 1] ? t.fi[t.rp[c]] : 0);
             t.pfw[size_t(c) * t.pw + e] = real ? t.fw[q] : 0.0;
         }
+    // longest run of coarse points whose fine points fit a restriction window
+    bool used = true;
+    for (int c = 0; c < nc; ++c) used = used && t.rp[c] < t.rp[c + 1];
+    for (int run = 64; run >= 32 && used && !t.run; --run) {
+        bool fits = true;
+        for (int c = 0; c < nc && fits; c += run) {
+            int lo = nf, hi = -1;
+            for (int q = t.rp[c]; q < t.rp[std::min(c + run, nc)]; ++q) {
+                lo = std::min(lo, t.fi[q]);
+                hi = std::max(hi, t.fi[q]);
+            }
+            fits = hi - lo < kRestrictWindow;
+        }
+        if (fits) t.run = run;
+    }
     return t;
 }
 
@@ -375,7 +390,7 @@ int helm3d_mg_create(int nlevels, helm3d_ctx* const* A, helm3d_ctx* const* S, he
             T.nf[a] = A[l]->n[a];
             T.nc[a] = A[l + 1]->n[a];
             T.ax[a] = MgAxis{di + o.I,  dd + o.wa,  dd + o.wb,  di + o.rp,
-                             di + o.fi, dd + o.fw, di + o.pfi, dd + o.pfw, tabs[size_t(l) * 3 + a].pw};
+                             di + o.fi, dd + o.fw, di + o.pfi, dd + o.pfw, tabs[size_t(l) * 3 + a].pw, tabs[size_t(l) * 3 + a].run};
         }
     }
     *out = mg;

@@ -270,8 +270,8 @@ __global__ __launch_bounds__(64) void gmres_lsq_kernel(const double* __restrict_
 // ||slot(K)||^2, summed here from the update pass's partials.  Reads skip, beta
 // and normr0, which no block of the launch writes; the decision for the next
 // cycle goes to stop.  The rows and the block's first points are loaded ahead
-// of the one-thread least squares, which takes most of the time (8211 points,
-// K = 5: 8.2 us for the one-block launch and 3.7 us for the update before).
+// of the one-thread least squares, which takes most of the time (18259 points,
+// K = 5: 6.9 us; before, 8.2 us for the one-block launch and 3.7 us for the update).
 template <typename R, int K>
 __global__ __launch_bounds__(KB) void cycle_end_kernel(const cpx<R>* __restrict__ V, long ldv,
                                                        const double* __restrict__ rows, int ldr, double tol,

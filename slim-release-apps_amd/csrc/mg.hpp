@@ -21,7 +21,12 @@ struct MgAxis {
     const int* pfi;
     const double* pfw;
     int pw;
+    // coarse points of which every run q * run .. (q + 1) * run - 1 (run <= 64)
+    // uses at most kRestrictWindow consecutive fine points; 0: fewer than 32,
+    // or a coarse point that no fine point uses
+    int run;
 };
+constexpr int kRestrictWindow = 128;
 
 struct MgAxes {
     int nf[3], nc[3];

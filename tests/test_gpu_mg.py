@@ -38,6 +38,26 @@ def test_transfers_match_oracle():
         assert np.linalg.norm(yc - (P.T @ xf) / 8) <= 1e-13 * np.linalg.norm(P.T @ xf / 8)
 
 
+# runs of 61 to 64 coarse points share a restriction window: widths around one,
+# two and four of them, the last run of one point; four fine planes per thread
+# of the prolongation and remainders
+@pytest.mark.parametrize("n", [(4, 4, 4), (109, 9, 8), (112, 6, 5), (116, 7, 6), (119, 8, 10), (238, 5, 7)])
+def test_transfer_runs(n):
+    import torch
+    from helm3d.mg import MLGMRES
+    v = np.full(int(np.prod(n)), 2000.0)
+    M = MLGMRES(v, n, 10.0, 4, 5.0, nlevels=2)
+    rng = np.random.default_rng(3)
+    nf, nc = M.grids[0]["nt"], M.grids[1]["nt"]
+    P = O.prolongation(nf, nc)
+    xc = rng.standard_normal(P.shape[1]) + 1j * rng.standard_normal(P.shape[1])
+    xf = rng.standard_normal(P.shape[0]) + 1j * rng.standard_normal(P.shape[0])
+    yf = M.transfer(0, torch.from_numpy(xc).cuda(), "prolong").cpu().numpy()
+    yc = M.transfer(0, torch.from_numpy(xf).cuda(), "restrict").cpu().numpy()
+    assert np.linalg.norm(yf - P @ xc) <= 1e-13 * np.linalg.norm(P @ xc)
+    assert np.linalg.norm(yc - (P.T @ xf) / 8) <= 1e-13 * np.linalg.norm(P.T @ xf / 8)
+
+
 @pytest.mark.parametrize("precision", ["c128", "mixed"])
 @pytest.mark.parametrize("mode", [1, 2])
 def test_mg_solve(mode, precision):
