@@ -48,10 +48,11 @@ class BatchSolver:
                  rows_per_thread=(1, 2)) -> dict:
         """Choose the stencil launch shape of a batch by timing a short batched
         solve (one restart cycle of two outer steps) for every candidate: 64 x 4
-        and 32 x 8 column tiles, 64 x 8 with two rows per thread, prefetch depth, and z chunks of nz/divisor for every operator.  The
-        fastest shape is left set on the operators; later solves converge to
-        the same tolerance whatever the shape (the fused BiCGStab partial sums
-        follow the shape, so iteration counts can move by a few)."""
+        and 32 x 8 column tiles, 64 x 8 with two rows per thread, prefetch
+        depth, and z chunks of nz/divisor for every operator.  The fastest
+        shape is left set on the operators; later solves converge to the same
+        tolerance whatever the shape (the fused BiCGStab partial sums follow
+        the shape, so iteration counts can move by a few)."""
         uniq = list({id(H): H for H in ops}.values())
         best = None
         for ty in tile_rows:
