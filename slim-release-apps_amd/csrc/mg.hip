@@ -212,7 +212,8 @@ hipError_t launch_prolong_add(const MgAxes& T, const cpx<R>* xc, cpx<R>* xf, hip
 template <typename R>
 hipError_t launch_restrict(const MgAxes& T, double scale, const cpx<R>* rf, cpx<R>* yc, hipStream_t s)
 {
-    if (T.ax[0].run > 0 && T.ax[1].pw <= 8) {
+    // grids of a ratio of 2 always fit; the gather takes the ratios beyond about 3
+    if (T.ax[0].run > 0 && T.ax[0].pw <= 8 && T.ax[1].pw <= 8) {
         const dim3 gw((T.nc[0] + T.ax[0].run - 1) / T.ax[0].run, (T.nc[1] + 3) / 4, T.nc[2]);
         if (T.ax[1].pw <= 4)
             hipLaunchKernelGGL((restrict_window_kernel<R, 4>), gw, dim3(KB), 0, s, T, scale, rf, yc);
