@@ -10,6 +10,10 @@
 // the textbook ratio rho'/rho; BICGSTAB.m:59 divides (rnew, r0_bar) by itself,
 // which makes beta = a/w -- that quirk is not reproduced.
 //
+// Here each update is a pass of its own.  The fused form of the stencil body
+// (epilogues 3 and 4) takes rho' from (rhat, s) - w (rhat, t) instead; the
+// kernels of this file that serve it are its start and its last z update.
+//
 // Scalar slots (doubles, device): see the BS_* offsets in bicgstab.hpp.
 #include "bicgstab.hpp"
 #include "kbody.hpp"

@@ -45,6 +45,9 @@ constexpr int kMaxChunk = 254;  // z planes per block (LDS holds their PML weigh
 template <typename R>
 __device__ inline cpx<R> zero() { return cpx<R>{R(0), R(0)}; }
 
+template <typename T, typename R>
+__device__ inline cpx<T> conv(cpx<R> a) { return cpx<T>{T(a.re), T(a.im)}; }
+
 // Output stores carry the non-temporal hint: no output is read again by the
 // launch that writes it, and streaming the outputs past the caches leaves
 // them to the halo planes of the inputs (the 240x240x140 matvec: 4-7 %
@@ -99,10 +102,15 @@ __device__ inline Cd cd_div(Cd a, Cd b)
 //      EPI 4 launch
 //   4: x = s = r - alpha v formed while staging, y = t = H s, partials
 //      (t, s), ||t||^2, (rhat, s) and (rhat, t)
+// U is the arithmetic of these updates: scalars, products and sums in U, every
+// stored or staged vector rounded to R once, as in the separate passes of
+// bicgstab.hip for U = double.  rho' is the product of rhat with the residual
+// ahead of its rounding, from sums in FP64.
 // 5 is an Arnoldi step (StepArgs X): EPI 0 with the scale summed from partials
 // and, after the march, the dots of the block's outputs with the basis.
 // The body runs one block `lin` of a launch of `G` blocks described by L.
-template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY = 1, int TXW = TX, int XG = TXW>
+template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY = 1, int TXW = TX, int XG = TXW,
+          typename U = R>
 __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int lin, const int G,
                                             const StepArgs<R>* X = nullptr)
 {
@@ -129,7 +137,7 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     // own point
     constexpr int kE3 = EPI == 3 ? 1 : 0;
     __shared__ cpx<R> sr[1 + kE3][1 + kE3 * (HY - 1)][1 + kE3 * (HX - 1)];
-    __shared__ cpx<R> sd[1 + kE3][1 + kE3 * (HY - 1)][1 + kE3 * (HX - 1)];
+    __shared__ cpx<U> sd[1 + kE3][1 + kE3 * (HY - 1)][1 + kE3 * (HX - 1)];
 
     const int nx = op.nx, ny = op.ny, nz = op.nz;
 
@@ -250,8 +258,8 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     // bt = beta, nbw = -beta omega, za = alpha, zw = omega; all zero on the
     // first iteration, whose p, v, t are zero and r = b).  EPI 4: s = r + ca v
     // (ca = -alpha).
-    cpx<R> ca = zero<R>();
-    cpx<R> na = zero<R>(), nw = zero<R>(), bt = zero<R>(), nbw = zero<R>(), za = zero<R>(), zw = zero<R>();
+    cpx<U> ca = zero<U>();
+    cpx<U> na = zero<U>(), nw = zero<U>(), bt = zero<U>(), nbw = zero<U>(), za = zero<U>(), zw = zero<U>();
     if constexpr (EPI == 3 || EPI == 4) {
         double* sc = L.sc;
         if constexpr (EPI == 3) {
@@ -269,12 +277,12 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
                     sc[BS_OMEGA] = w.re;
                     sc[BS_OMEGA + 1] = w.im;
                 }
-                na = cpx<R>{R(-a.re), R(-a.im)};
-                nw = cpx<R>{R(-w.re), R(-w.im)};
-                bt = cpx<R>{R(beta.re), R(beta.im)};
-                nbw = cpx<R>{R(-bw.re), R(-bw.im)};
-                za = cpx<R>{R(a.re), R(a.im)};
-                zw = cpx<R>{R(w.re), R(w.im)};
+                na = cpx<U>{U(-a.re), U(-a.im)};
+                nw = cpx<U>{U(-w.re), U(-w.im)};
+                bt = cpx<U>{U(beta.re), U(beta.im)};
+                nbw = cpx<U>{U(-bw.re), U(-bw.im)};
+                za = cpx<U>{U(a.re), U(a.im)};
+                zw = cpx<U>{U(w.re), U(w.im)};
             }
         } else {
             const Cd a = cd_div(cd_ld(sc, L.rho_new), cd_ld(sc, BS_RV));
@@ -282,14 +290,18 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
                 L.sc[BS_ALPHA] = a.re;
                 L.sc[BS_ALPHA + 1] = a.im;
             }
-            ca = cpx<R>{R(-a.re), R(-a.im)};
+            ca = cpx<U>{U(-a.re), U(-a.im)};
         }
     }
     // EPI 3/4: staged x at the own points of the previous plane; EPI 3: r'
     // and dz there
-    cpx<R> Xlast[RY], Rlast[RY], Dlast[RY];
+    cpx<R> Xlast[RY], Rlast[RY];
+    cpx<U> Dlast[RY];
 #pragma unroll
-    for (int r = 0; r < RY; ++r) Xlast[r] = Rlast[r] = Dlast[r] = zero<R>();
+    for (int r = 0; r < RY; ++r) {
+        Xlast[r] = Rlast[r] = zero<R>();
+        Dlast[r] = zero<U>();
+    }
     // output scale: alpha, or alpha / sqrt(*anrm) with the norm held on the device
     R alpha = (EPI <= 1 && L.anrm) ? R(double(L.alpha) / sqrt(*L.anrm)) : L.alpha;
 
@@ -372,15 +384,16 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
             const bool v = inz && sin_[t];
             cpx<R> xv = S.x[t];
             if constexpr (EPI == 3) {
-                const cpx<R> sv = cfma(S.x[t], na, S.f[t]);
-                const cpx<R> rv = cfma(sv, nw, S.g[t]);
-                xv = cfma(cfma(rv, bt, S.e[t]), nbw, S.f[t]);
+                const cpx<U> pu = conv<U>(S.e[t]), vu = conv<U>(S.f[t]);
+                const cpx<U> sv = conv<U>(conv<R>(cfma(conv<U>(S.x[t]), na, vu)));
+                const cpx<R> rv = conv<R>(cfma(sv, nw, conv<U>(S.g[t])));
+                xv = conv<R>(cfma(cfma(conv<U>(rv), bt, pu), nbw, vu));
                 if (shas[t]) {
                     sr[buf][sys[t]][sxs[t]] = rv;
-                    sd[buf][sys[t]][sxs[t]] = cfma(cmul(za, S.e[t]), zw, sv);
+                    sd[buf][sys[t]][sxs[t]] = cfma(cmul(za, pu), zw, sv);
                 }
             } else if constexpr (EPI == 4) {
-                xv = cfma(xv, ca, S.e[t]);
+                xv = conv<R>(cfma(conv<U>(xv), ca, conv<U>(S.e[t])));
             }
             xs[t] = v ? xv : zero<R>();
             if (shas[t]) su[buf][sys[t]][sxs[t]] = xs[t];
@@ -592,7 +605,7 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
                 st_out(dy, out);
                 st_out(d2, Xlast[r]);
                 st_out(d3, Rlast[r]);
-                st_out(d4, zo[r] + Dlast[r]);
+                st_out(d4, conv<R>(conv<U>(zo[r]) + Dlast[r]));
                 if (live) {
                     // (rhat, v) += conj(rhat) v
                     acc[0] += double(bb[r].re) * double(out.re) + double(bb[r].im) * double(out.im);

@@ -1,6 +1,11 @@
 // The two operator applications of a complex64 BiCGStab iteration with every
 // vector update fused in (epilogues 3 and 4 of the stencil body), for one
-// vector: the work-list form of helm27_batch.hip without the list.
+// vector: the work-list form of helm27_batch.hip without the list, with the
+// updates and their scalars in FP64 and one rounding per stored vector, as the
+// separate passes of bicgstab.hip have them (the batch rounds every product).
+// An outer step of 25 iterations: 97 x 72 x 50 0.88 ms, 161 x 150 x 100 2.97,
+// 240 x 240 x 140 6.9; with the updates in FP32 0.87, 2.95 and 6.8, with
+// separate passes 1.44, 3.32 and 8.8.
 #include "helm27_body.hpp"
 
 namespace helm3d {
@@ -15,7 +20,7 @@ constexpr int kFTx = 32, kFTy = 8, kFPf = 2;
 template <bool ADJ, bool WNC, int EPI>
 __global__ __launch_bounds__(kFTx* kFTy) void helm27_fused_kernel(StencilLaunch<float> L)
 {
-    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1, kFTx>(L, blockIdx.x, gridDim.x);
+    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1, kFTx, kFTx, double>(L, blockIdx.x, gridDim.x);
 }
 
 template <bool A, bool W, int EPI>
