@@ -155,9 +155,13 @@ int helm3d_apply_noalloc(int variant, const int n[3], const double h[3], const i
 /* Stencil launch shape: z planes per block (0: automatic), column-tile rows
  * (4 or 8), planes of loads in flight (1 to 4; the batched kernels use at
  * most 2) and rows per thread (1: tiles of 32 columns, 64 by 4 rows in the
- * batched kernels; or 2 with 8 tile rows: tiles of 64 columns).  The result
- * is identical for every shape; only speed changes.  Chosen per grid
- * by the autotuner (helm3d_autotune). */
+ * batched kernels; or 2 with 8 tile rows: tiles of 64 columns).  The product
+ * is identical for every shape, in the batched kernels too; only speed
+ * changes.  Chosen per grid by the autotuner (helm3d_autotune).  Sums that a
+ * launch takes over its blocks (residual norms, the dot products of a mixed
+ * batch) group their terms by the shape.  The fixed-length inner solve of
+ * helm3d_solve_mixed and the short Arnoldi steps of the multigrid hierarchies
+ * always take the automatic shape, so that they depend on the grid alone. */
 int helm3d_set_launch(helm3d_ctx *ctx, int kchunk, int tile_rows, int prefetch, int rows_per_thread);
 int helm3d_get_launch(helm3d_ctx *ctx, int *kchunk, int *tile_rows, int *prefetch, int *rows_per_thread,
                       int *blocks);
@@ -169,7 +173,8 @@ int helm3d_get_launch(helm3d_ctx *ctx, int *kchunk, int *tile_rows, int *prefetc
  * `reps` launches each with HIP events on the context's stream, and keeps the
  * fastest (results are identical for every shape).  No counterpart in the
  * reference; the batched solves use each item's tuned z chunk and the first
- * item's tile rows, rows per thread and prefetch. */
+ * item's tile rows, rows per thread and prefetch (its automatic shape where
+ * none was chosen). */
 int helm3d_autotune(helm3d_ctx *ctx, int mode, int precision, int reps, int *kchunk, int *tile_rows,
                     int *prefetch, int *rows_per_thread, double *best_ms);
 

@@ -12,9 +12,10 @@ namespace {
 // active[it] == 0 are skipped.  MIX: items marked narrow take tiles of half the
 // columns and twice the rows (the same threads), the others TX x TY ones; a
 // wave of a narrow tile is two rows, so only the y multipliers leave the scalar
-// registers.  The choice is per item and per block, so an item's bits do not
-// depend on its neighbours in the list, and the wide items of a mixed launch
-// take as long as in a launch of their own.
+// registers.  The choice is per item and per block, and the wide items of a
+// mixed launch take as long as in a launch of their own.  The product at a point
+// is the same for every shape; the partial sums of EPI 3 and 4 follow the
+// item's blocks.
 template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY, bool MIX, int TXW>
 __global__ __launch_bounds__(TXW* TY / RY) void helm27_batch_kernel(const StencilLaunch<R>* __restrict__ items,
                                                               const int* __restrict__ first, int nitems,

@@ -20,7 +20,7 @@ constexpr int kFTx = 32, kFTy = 8, kFPf = 2;
 template <bool ADJ, bool WNC, int EPI>
 __global__ __launch_bounds__(kFTx* kFTy) void helm27_fused_kernel(StencilLaunch<float> L)
 {
-    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1, kFTx, kFTx, double>(L, blockIdx.x, gridDim.x);
+    helm27_body<float, ADJ, false, WNC, kFTy, kFPf, EPI, 1, kFTx, double>(L, blockIdx.x, gridDim.x);
 }
 
 template <bool A, bool W, int EPI>

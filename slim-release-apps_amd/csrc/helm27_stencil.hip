@@ -36,7 +36,7 @@ namespace {
 template <typename R, bool ADJ, bool DERIV, bool WNC, int TY, int PF, int EPI, int RY, int TXW>
 __global__ __launch_bounds__(TXW* TY / RY) void helm27_kernel(StencilLaunch<R> L)
 {
-    helm27_body<R, ADJ, DERIV, WNC, TY, PF, EPI, RY, TXW, 32>(L, blockIdx.x, gridDim.x);
+    helm27_body<R, ADJ, DERIV, WNC, TY, PF, EPI, RY, TXW>(L, blockIdx.x, gridDim.x);
 }
 
 }  // namespace

@@ -299,3 +299,58 @@ def test_uneven_workload_chunked():
     x1, i1 = S.solve(ops, bs, method="mixed", tol=1e-6, inner_maxit=10)
     for a, b_, ia, ib in zip(xs, x1, infos, i1):
         assert ia.iters == ib.iters and torch.equal(a, b_)
+
+
+SHAPES = [(0, 4, 1, 1), (7, 4, 2, 1), (0, 8, 2, 1), (9, 8, 1, 1), (0, 8, 2, 2), (5, 8, 1, 2)]
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("wnc", [False, True])
+@pytest.mark.parametrize("n", [(95, 33, 21), (100, 30, 20)])
+def test_batch_product_same_for_every_shape(n, wnc, mode):
+    """One cycle of a plain batch from x = 0 takes nothing from the launch shape
+    but the products (its dots and norms are passes of their own, grouped by
+    the grid alone), so the solutions have to be equal in every bit: untuned
+    (32 x 8 tiles for nx = 95, 64 x 4 for 100), every tile shape, and an untuned
+    item behind a tuned first one and the other way round.  Columns 32 to 63
+    lie inside the PML faces, columns 0 to 31 do not."""
+    import torch
+    from helm3d import BatchSolver, Helm3d
+    print(f"batch shapes n={n} wnc={wnc} mode={mode}", flush=True)
+    rng = np.random.default_rng(31)
+    N = int(np.prod(n))
+    wn = rng.uniform(2e-4, 2e-3, N) * ((1.0 + 0.02j) if wnc else 1.0)
+    dev = torch.device("cuda:0")
+    op = lambda: Helm3d(n, (10.0,) * 3, np.full((2, 3), 6), torch.from_numpy(wn).to(dev))  # noqa: E731
+    b = torch.from_numpy(rng.standard_normal(N) + 1j * rng.standard_normal(N)).to(dev)
+    S = BatchSolver(dev)
+    run = lambda ops: S.solve(ops, [b] * len(ops), mode=mode, method="plain", tol=1e-30, maxinnerit=6,  # noqa: E731
+                              maxit=1)[0]
+    plain, tuned = op(), op()
+    want = run([plain])[0]
+    assert float(want.norm()) > 0.0
+    for shape in SHAPES:
+        tuned.set_launch(*shape)
+        for ops in ([tuned], [tuned, plain], [plain, tuned]):
+            for x in run(ops):
+                assert torch.equal(x, want), (shape, len(ops))
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_mixed_batch_tuned_and_untuned_items(shape):
+    """A mixed batch of an item with a chosen launch shape and one without, in
+    both orders (the first item's shape governs): all reach tol."""
+    import torch
+    from helm3d import BatchSolver
+    c1, w1, H1 = _op((83, 20, 14), 6, 5.0, 12)
+    c2, w2, H2 = _op((40, 28, 30), 6, 6.0, 13)
+    H2.set_launch(*shape)
+    items = [(c1, w1, H1, (16, 16, 3)), (c2, w2, H2, (20, 14, 3))]
+    S = BatchSolver("cuda:0")
+    for it in (items, items[::-1]):
+        print("tuned and untuned", shape, it[0][0].nt, flush=True)
+        bs = [_rhs(c, s) for c, _, _, s in it]
+        xs, infos = S.solve([i[2] for i in it], [torch.from_numpy(b).cuda() for b in bs], method="mixed", tol=1e-6,
+                            inner_maxit=10)
+        for (c, w, _, _), b, x, inf in zip(it, bs, xs, infos):
+            assert inf.converged and _relres(c, w, b, x.cpu().numpy(), 1) < 1e-6
