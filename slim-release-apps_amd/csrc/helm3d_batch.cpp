@@ -137,17 +137,32 @@ T* at(helm3d_batch* b, size_t off) { return reinterpret_cast<T*>(static_cast<cha
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 // Work lists of unchosen shape take tiles of 32 columns by 8 rows on grids whose
-// last 64-column tile would be half empty, 64 by 4 on the others (the rule
-// looks at the item alone).  Four mixed solves of nx x 72 x 50: nx = 84 9.09 ->
-// 7.85 ms, 65 8.78 -> 7.81, 130 11.74 -> 10.19, 160 x 160 x 60 23.9 -> 21.9;
-// where the last tile is filled narrow tiles read more halo lines: 97 9.23 ->
-// 9.97, 128 9.51 -> 9.53, 240 x 240 x 60 44.3 -> 45.2.
-bool narrow_tiles(int nx) { return (((nx + 31) / 32) & 1) != 0; }
+// last 64-column tile would be half empty, up to 224 columns, 64 by 4 on the
+// others (the rule looks at the item alone).  Four mixed solves of nx x 72 x 50:
+// nx = 84 9.09 -> 7.85 ms, 65 8.78 -> 7.81, 130 11.74 -> 10.19, 160 x 160 x 60
+// 23.9 -> 21.9; an outer step of four 224 x 180 x 100 items 21.8 -> 20.6.  Where
+// the last tile is filled narrow tiles read more halo lines, nx = 97 9.23 ->
+// 9.97, 240 x 240 x 60 44.3 -> 45.2, and beyond 256 columns the half tile they
+// save is no longer worth those: 262 x 273 x 148 62.7 -> 66.5, 330 x 200 x 120
+// 35.6 -> 36.7.
+bool narrow_tiles(int nx)
+{
+    const int w = (nx + 31) / 32;
+    return (w & 1) != 0 && w < 9;
+}
 
-// z planes per block of an item: the chosen launch shape, or the chunk for a
-// launch that holds four such items (an item's partial sums follow its chunk,
-// so the chunk must not depend on what else is in the batch).  One 48 x 48 x 40
-// grid with two right-hand sides: 4 planes 3.5 ms, 8 planes 4.3.
+// z planes per block of an item: the chosen launch shape, or by rule.  An
+// item's partial sums follow its chunk, so the chunk must not depend on what
+// else is in the batch and has to do for one item as for thirty.  The cost model
+// is asked for a launch of four such items, with two exceptions:
+// * below 32 tiles no more than 8 planes: 84 x 72 x 50, two outer steps of 1 / 4
+//   / 16 items: 14 planes 2.39 / 3.32 / 9.17 ms, 8 planes 1.88 / 3.05 / 9.10;
+// * from 240 to 479 tiles, where one item in two chunks fills the chip, two
+//   chunks: 240 x 240 x 140 x 8: 48 planes 78.2 ms, 70 planes 75.8.
+// Elsewhere the model weighs few items against many: against about 480 blocks
+// an item it gains 9 % on 120 x 90 x 60 x 8 (8.4 ms, 9.2) and 20 % on one or two
+// 48 x 48 x 40 items (1.40, 1.75), and loses 8 % on one 128 x 128 x 80 item (3.1,
+// 2.8) and 14 % on sixteen 48 x 48 x 40 ones (4.3, 3.75).
 StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, int ry, bool mix)
 {
     if (mix) {
@@ -159,8 +174,11 @@ StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, int ry, bool mix)
     int kc = c->grid.kchunk;
     if (c->grid_auto) {
         const StencilGrid g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], 1, ty, pf, ry, tx);
-        const long tiles = 4L * g.tiles_x * g.tiles_y;
-        kc = stencil_chunk(&tiles, &c->n[2], 1, kSlots64);
+        const int tiles = g.tiles_x * g.tiles_y, nz = c->n[2];
+        const long four = 4L * tiles;
+        kc = stencil_chunk(&four, &nz, 1, kSlots64);
+        if (tiles < 32) kc = std::min(kc, 8);
+        else if (tiles >= 240 && tiles < 480) kc = (nz + 1) / 2;
     }
     return stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, ry, tx);
 }
