@@ -149,6 +149,8 @@ struct helm3d_ctx {
     // the shapes by rule, kept for launches whose block sums reach the result
     // (the Arnoldi steps of short vectors): their bits follow the grid alone
     StencilGrid rule64{}, rule32{};
+    // the fused BiCGStab forms of a single mixed solve, by rule as well
+    StencilGrid fused{};
 
     double* part = nullptr;
     size_t part_cap = 0;
@@ -335,8 +337,8 @@ constexpr long kMaxDeviceCycles = 16;
 // mirror) and the stencil's write-only sink.
 inline int ensure_work(helm3d_ctx* c)
 {
-    const size_t nblk = std::max<size_t>(
-        std::max(std::max(c->grid.blocks, c->grid32.blocks), std::max(c->rule64.blocks, c->rule32.blocks)), kMaxPartials);
+    const size_t nblk = std::max<size_t>({size_t(kMaxPartials), size_t(c->grid.blocks), size_t(c->grid32.blocks),
+                                          size_t(c->rule64.blocks), size_t(c->rule32.blocks), size_t(c->fused.blocks)});
     CHK(ensure_t(&c->part, &c->part_cap, nblk * 2 * kMaxBasis));
     CHK(ensure_t(&c->small, &c->small_cap, 2 * kMaxBasis + 8));
     CHK(ensure(&c->sink, &c->sink_cap, size_t(kSinkSlots) * sizeof(cpx<double>)));

@@ -86,22 +86,28 @@ struct StencilGrid {
     int tiles_x, tiles_y, kchunk, nchunks, blocks, ty, pf, ry, tx;
 };
 
-// z planes per block (even) for a launch over columns of `tiles[i]` tiles and
-// nz[i] planes, i < n.  A block marches its planes and two halo planes, blocks
-// run `slots` at a time, and the launch ends with a tail in which slots idle,
-// longer when the last round is nearly empty:
-//   cost(kc) = planes(kc) / slots + (kc + 2) (0.2 + 0.15 (ceil(x) - x)),
-//   planes = sum tiles (nz + 2 chunks), x = blocks / slots,
-// fitted to launches of chunks from 2 planes to the whole column on single
-// grids of 48 x 48 x 40 to 296 x 296 x 168 and on batches of 2 to 8 of them;
-// the chunk it picks is within 8 % of the best of the sweep on each
-// (complex128 48 x 48 x 40: 2 planes 5.9 us, 7 planes 9.7; 84^3: 6 planes 12.6,
-// 9 planes 16.3, 42 planes 34.0; complex64 240 x 240 x 140: 18 planes 45.3, 70
-// planes 56.8; six uneven grids together: 16 planes 13.7 ms, 8 planes 15.1).
-// About two complex128 blocks of 256 threads fit a compute unit, four
-// complex64 ones.
-int stencil_chunk(const long* tiles, const int* nz, int n, int slots);
-constexpr int kSlots64 = 512, kSlots32 = 1024;
+// z planes per block (even) for a launch over `tiles` columns of nz planes.  A
+// block marches its planes and two halo planes, blocks run `slots` at a time,
+// and the launch ends with a tail in which slots idle, longer when the last
+// round is nearly empty:
+//   cost(kc) = tiles (nz + halo chunks) / slots
+//            + (kc + fill) (wait + tail (ceil(x) - x)),  x = blocks / slots,
+// fitted to launches of chunks from 2 planes to the whole column on 36 grids of
+// 31 x 31 x 19 to 420 x 400 x 150 with rotating inputs (complex128 48 x 48 x 40:
+// 2 planes 6.0 us, 8 planes 9.7; 84^3: 6 planes 11.9, 9 planes 16.3, 42 planes
+// 34.0).  In complex128 the same constants do not serve both ends: three blocks
+// of 256 threads fit a compute unit, and grids of more than 100 tiles want longer
+// chunks than a fit over all finds (best of the sweep 100 %: 187 x 203 x 111 20
+// planes 108 %, 28 planes 105; 200 x 200 x 100 20 planes 113, 26 planes 100; 240
+// x 240 x 140 24 planes 105, 48 planes 100; mean over 16 such grids 105.5 and
+// 101.5).
+struct ChunkCost {
+    int slots;
+    double halo, fill, wait, tail;
+};
+constexpr ChunkCost kCost64{512, 2, 2, 0.2, 0.15}, kCost64Large{768, 4, 0, 0.15, 0.15}, kCost32{1024, 2, 2, 0.2, 0.15};
+constexpr int kLargeTiles = 100;
+int stencil_chunk(long tiles, int nz, const ChunkCost& m);
 
 // kchunk <= 0 picks the chunk by stencil_chunk for precision R; ty in {4, 8};
 // pf in 1..4; ry in {1, 2} (2 needs ty = 8; otherwise 1 is used); tx = 0: tiles

@@ -41,22 +41,16 @@ __global__ __launch_bounds__(TXW* TY / RY) void helm27_kernel(StencilLaunch<R> L
 
 }  // namespace
 
-int stencil_chunk(const long* tiles, const int* nz, int n, int slots)
+int stencil_chunk(long tiles, int nz, const ChunkCost& m)
 {
-    int top = 1;
-    for (int i = 0; i < n; ++i) top = std::max(top, nz[i]);
-    top = std::min(top, kMaxChunk);
+    const int top = std::min(nz, kMaxChunk);
     int best = top;
     double best_cost = 1e300;
     for (int kc = 2; kc < top + 2; kc += 2) {
-        double blocks = 0.0, planes = 0.0;
-        for (int i = 0; i < n; ++i) {
-            const int ch = (nz[i] + kc - 1) / kc;
-            blocks += double(tiles[i]) * ch;
-            planes += double(tiles[i]) * (nz[i] + 2 * ch);
-        }
-        const double x = blocks / slots;
-        const double cost = planes / slots + (std::min(kc, top) + 2) * (0.2 + 0.15 * (std::ceil(x) - x));
+        const int chunks = (nz + kc - 1) / kc;
+        const double x = double(tiles) * chunks / m.slots;
+        const double cost = tiles * (nz + m.halo * chunks) / m.slots +
+                            (std::min(kc, top) + m.fill) * (m.wait + m.tail * (std::ceil(x) - x));
         if (cost < best_cost) {
             best_cost = cost;
             best = std::min(kc, top);
@@ -77,7 +71,9 @@ StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty, int pf, int
     g.tiles_y = (ny + g.ty - 1) / g.ty;
     if (kchunk <= 0) {
         const long tiles = long(g.tiles_x) * g.tiles_y;
-        kchunk = stencil_chunk(&tiles, &nz, 1, std::is_same<R, double>::value ? kSlots64 : kSlots32);
+        const ChunkCost& m =
+            !std::is_same<R, double>::value ? kCost32 : (tiles > kLargeTiles ? kCost64Large : kCost64);
+        kchunk = stencil_chunk(tiles, nz, m);
     }
     g.kchunk = std::max(1, std::min(std::min(kchunk, nz), kMaxChunk));
     g.nchunks = (nz + g.kchunk - 1) / g.kchunk;

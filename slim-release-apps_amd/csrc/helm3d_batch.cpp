@@ -175,8 +175,7 @@ StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, int ry, bool mix)
     if (c->grid_auto) {
         const StencilGrid g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], 1, ty, pf, ry, tx);
         const int tiles = g.tiles_x * g.tiles_y, nz = c->n[2];
-        const long four = 4L * tiles;
-        kc = stencil_chunk(&four, &nz, 1, kSlots64);
+        kc = stencil_chunk(4L * tiles, nz, kCost64);
         if (tiles < 32) kc = std::min(kc, 8);
         else if (tiles >= 240 && tiles < 480) kc = (nz + 1) / 2;
     }

@@ -641,10 +641,7 @@ int bicgstab_fixed(helm3d_ctx* c, hipStream_t st, int variant, const cpx<float>*
     cpx<float>* p[2] = {W + 2 * ld, W + 3 * ld};
     cpx<float>* v[2] = {W + 4 * ld, W + 5 * ld};
     cpx<float>* t = W + 6 * ld;
-    // the fused forms hold two to four vectors a point and fit a compute unit
-    // as often as the complex128 kernel: its chunk (97 x 79 x 65: 34.8 ms a
-    // solve, 36.6 with the chunk of the plain complex64 kernel)
-    const StencilGrid& G = c->rule64;
+    const StencilGrid& G = c->fused;
     const int nblk = krylov_blocks(N);
     double* sc = c->bsc;
     HIPCHK(launch_bicg_init(b, p[0], v[0], t, z, N, c->part, nblk, st));
@@ -887,6 +884,13 @@ int helm3d_set_model(helm3d_ctx* c, const int n[3], const double h[3], const int
     if (!same_grid) {
         c->grid = c->rule64 = stencil_grid<double>(n[0], n[1], n[2], 0);
         c->grid32 = c->rule32 = stencil_grid<float>(n[0], n[1], n[2], 0);
+        // the fused forms hold two to four vectors a point and fit a compute
+        // unit as often as the complex128 kernel: its cost model (97 x 79 x 65:
+        // 34.8 ms a solve, 36.6 with the chunk of the plain complex64 kernel);
+        // the constants for large complex128 grids win and lose here (20 inner
+        // iterations: 220 x 180 x 120 3.45 -> 3.67 ms, 130 x 240 x 90 2.65 -> 2.40)
+        const long tiles = long(c->rule64.tiles_x) * c->rule64.tiles_y;
+        c->fused = stencil_grid<float>(n[0], n[1], n[2], stencil_chunk(tiles, n[2], kCost64));
         c->grid_auto = true;
     }
     CHK(ensure_work(c));
