@@ -16,7 +16,6 @@
 //    Each output row is a gather, so the kernel needs no atomics; the host
 //    builds the transposed rows for the injection direction.
 #include <algorithm>
-#include <type_traits>
 
 #include "fwi.hpp"
 
@@ -189,39 +188,100 @@ __global__ __launch_bounds__(KB) void extension_adjoint_kernel(ExtGrid G, const 
     }
 }
 
-// LPR lanes per stored row (a power of two up to a wave): the entries of a
-// row are strided over its lanes and the lane sums added by a tree.
-template <int LPR>
-__global__ __launch_bounds__(KB) void csr_apply_kernel(int nrows, const long long* __restrict__ rowptr,
-                                                       const long long* __restrict__ col,
-                                                       const double* __restrict__ w,
-                                                       const long long* __restrict__ oidx, double alpha,
-                                                       const cpx<double>* __restrict__ in,
-                                                       cpx<double>* __restrict__ out, int accumulate)
+__device__ inline void csr_store(cpx<double>* out, long long o, double alpha, double re, double im, int accumulate)
 {
-    const long t = long(blockIdx.x) * KB + threadIdx.x;
-    const long r = t / LPR;
-    if (r >= nrows) return;  // uniform over a row's lanes
-    const int lane = int(t % LPR);
+    cpx<double> y{alpha * re, alpha * im};
+    if (accumulate) {
+        const cpx<double> p = out[o];
+        y.re += p.re;
+        y.im += p.im;
+    }
+    out[o] = y;
+}
+
+// One wave per stored row: the entries are strided over its lanes and the lane
+// sums added by a tree.
+__global__ __launch_bounds__(KB) void csr_row_kernel(int nrows, const long long* __restrict__ rowptr,
+                                                     const long long* __restrict__ col,
+                                                     const double* __restrict__ w,
+                                                     const long long* __restrict__ oidx, double alpha,
+                                                     const cpx<double>* __restrict__ in,
+                                                     cpx<double>* __restrict__ out, int accumulate)
+{
+    const long r = long(blockIdx.x) * (KB / 64) + (threadIdx.x >> 6);
+    if (r >= nrows) return;
+    const int lane = threadIdx.x & 63;
     double re = 0.0, im = 0.0;
-    for (long long e = rowptr[r] + lane; e < rowptr[r + 1]; e += LPR) {
+    for (long long e = rowptr[r] + lane; e < rowptr[r + 1]; e += 64) {
         const cpx<double> v = in[col[e]];
         re += w[e] * v.re;
         im += w[e] * v.im;
     }
+    re = wave_sum_d(re);
+    im = wave_sum_d(im);
+    if (lane == 0) csr_store(out, oidx ? oidx[r] : r, alpha, re, im, accumulate);
+}
+
+// `per` (at most 64) consecutive stored rows per wave, lane l holding the ends
+// of row l and, in the end, its sum.  How the wave works follows from its
+// longest row: a lane per row up to 4 entries, 8 lanes per row up to 64, else
+// the whole wave, row after row.
+template <int L>
+__device__ inline void csr_rows_by(int nr, int lane, long long e0, long long e1, const long long* __restrict__ col,
+                                   const double* __restrict__ w, const cpx<double>* __restrict__ in, double& re,
+                                   double& im)
+{
+    constexpr int G = 64 / L;  // rows at a time; those behind row nr - 1 are empty
+    for (int q = 0; q < nr; q += G) {
+        const int row = min(q + lane / L, 63);
+        const long long b = __shfl(e0, row, 64), e = __shfl(e1, row, 64);
+        double sr = 0.0, si = 0.0;
+        for (long long t = b + lane % L; t < e; t += L) {
+            const cpx<double> v = in[col[t]];
+            sr += w[t] * v.re;
+            si += w[t] * v.im;
+        }
 #pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) {
-        re += __shfl_xor(re, o, LPR);
-        im += __shfl_xor(im, o, LPR);
+        for (int o = L / 2; o > 0; o >>= 1) {
+            sr += __shfl_xor(sr, o, 64);
+            si += __shfl_xor(si, o, 64);
+        }
+        const int k = lane - q;  // lane q + k takes the sum of the k-th group
+        const double gr = __shfl(sr, (k * L) & 63, 64), gi = __shfl(si, (k * L) & 63, 64);
+        if (k >= 0 && k < G) {
+            re = gr;
+            im = gi;
+        }
     }
-    if (lane != 0) return;
-    const long long o = oidx ? oidx[r] : r;
-    cpx<double> y{alpha * re, alpha * im};
-    if (accumulate) {
-        y.re += out[o].re;
-        y.im += out[o].im;
+}
+
+__global__ __launch_bounds__(KB) void csr_rows_kernel(int nrows, int per, const long long* __restrict__ rowptr,
+                                                      const long long* __restrict__ col,
+                                                      const double* __restrict__ w,
+                                                      const long long* __restrict__ oidx, double alpha,
+                                                      const cpx<double>* __restrict__ in,
+                                                      cpx<double>* __restrict__ out, int accumulate)
+{
+    const int lane = threadIdx.x & 63;
+    const long r0 = (long(blockIdx.x) * (KB / 64) + (threadIdx.x >> 6)) * per;
+    if (r0 >= nrows) return;
+    const int nr = int(min(long(per), nrows - r0));
+    long long e0 = 0, e1 = 0;
+    if (lane < nr) {
+        e0 = rowptr[r0 + lane];
+        e1 = rowptr[r0 + lane + 1];
     }
-    out[o] = y;
+    const long long len = e1 - e0;
+    double re = 0.0, im = 0.0;
+    if (__any(len > 64)) csr_rows_by<64>(nr, lane, e0, e1, col, w, in, re, im);
+    else if (__any(len > 4)) csr_rows_by<8>(nr, lane, e0, e1, col, w, in, re, im);
+    else
+        for (long long e = e0; e < e1; ++e) {
+            const cpx<double> v = in[col[e]];
+            re += w[e] * v.re;
+            im += w[e] * v.im;
+        }
+    if (lane < nr) csr_store(out, oidx ? oidx[r0 + lane] : r0 + lane, alpha, re, im, accumulate);
 }
 
 int grid_blocks(long n) { return int(std::min<long>(std::max<long>((n + KB - 1) / KB, 1), 8192)); }
@@ -251,26 +311,29 @@ hipError_t launch_extension_adjoint(const ExtGrid& G, const double* gpml, double
     return hipGetLastError();
 }
 
-// Lanes per row by the row count alone (the entry counts are on the device):
-// with few rows (receiver sampling, 512 entries a row off the grid) the chip
-// is idle and a wave per row hides the chain of a long row; with many
-// (injection onto the grid, mostly one entry a row) a lane per row is enough.
-// 400 rows of 512 entries: 413 us with a lane per row, 12 us with a wave.
+// The host knows the row count, not the entry counts (they are on the device).
+// Up to 4096 rows the chip is idle enough for a wave per row (receiver sampling,
+// 512 entries a row off the grid: 400 rows 4.5 us, 4096 rows 16.3; a lane per row
+// 325 and 333), one entry a row costing 2.4 us at 1000 rows and 3.2 at 4096 (a
+// lane per row 2.4).  More rows go to about 3072 waves that look at their rows:
+// 16384 rows of 1 / 64 / 512 entries 2.4 / 11.3 / 60.7 us, a lane per row 2.3 /
+// 44.5 / 398, a wave per row 6.4 / 10.7 / 55.6.
 hipError_t launch_csr_apply(int nrows, const long long* rowptr, const long long* col, const double* w,
                             const long long* oidx, double alpha, const cpx<double>* in, cpx<double>* out,
                             bool accumulate, hipStream_t s)
 {
     if (nrows <= 0) return hipSuccess;
-    auto go = [&](auto lpr) {
-        constexpr int L = decltype(lpr)::value;
-        const long blocks = (long(nrows) * L + KB - 1) / KB;
-        hipLaunchKernelGGL((csr_apply_kernel<L>), dim3(unsigned(blocks)), dim3(KB), 0, s, nrows, rowptr, col, w, oidx,
-                           alpha, in, out, int(accumulate));
+    constexpr int kWaves = KB / 64;
+    if (nrows <= 4096) {
+        hipLaunchKernelGGL(csr_row_kernel, dim3((nrows + kWaves - 1) / kWaves), dim3(KB), 0, s, nrows, rowptr, col, w,
+                           oidx, alpha, in, out, int(accumulate));
         return hipGetLastError();
-    };
-    if (nrows <= 16384) return go(std::integral_constant<int, 64>{});
-    if (nrows <= 65536) return go(std::integral_constant<int, 8>{});
-    return go(std::integral_constant<int, 1>{});
+    }
+    const int per = std::min(64, (nrows - 1) / 3072 + 1);
+    const int waves = (nrows - 1) / per + 1;
+    hipLaunchKernelGGL(csr_rows_kernel, dim3((waves - 1) / kWaves + 1), dim3(KB), 0, s, nrows, per, rowptr, col, w,
+                       oidx, alpha, in, out, int(accumulate));
+    return hipGetLastError();
 }
 
 }  // namespace helm3d

@@ -325,3 +325,39 @@ def test_sparse_rows_lanes(rows, per):
     Helm3d(device="cuda:0").csr_apply(SparseRows(A, "cuda:0"), torch.from_numpy(x).cuda(), out, alpha=0.5,
                                       accumulate=True)
     assert relerr(out.cpu().numpy(), y0 + 0.5 * (A @ x)) <= 1e-13
+
+
+@pytest.mark.parametrize("rows", [4096, 4097, 6145, 200001])
+@pytest.mark.parametrize("longest", [1, 4, 5, 64, 65, 300])
+def test_sparse_rows_uneven(rows, longest):
+    """Stored rows of 0 to `longest` entries (every 997th as long as that): a
+    wave per row up to 4096 rows, beyond that up to 64 rows a wave with a lane,
+    8 lanes or the wave for each, by the longest row of the wave."""
+    from types import SimpleNamespace
+    import scipy.sparse as sp
+    import torch
+    from helm3d import Helm3d
+    print(f"csr rows={rows} longest={longest}", flush=True)
+    rng = np.random.default_rng(rows + longest)
+    count = rng.integers(0, min(longest, 6) + 1, rows)
+    count[::997] = longest
+    count[-1] = longest
+    rowptr = np.concatenate([[0], np.cumsum(count)])
+    cols, w = rng.integers(0, 1000, rowptr[-1]), rng.standard_normal(rowptr[-1])
+    A = sp.csr_matrix((w, cols, rowptr), shape=(rows, 1000))
+    x = rng.standard_normal(1000) + 1j * rng.standard_normal(1000)
+    y0 = rng.standard_normal(rows) + 1j * rng.standard_normal(rows)
+    oidx = rng.permutation(rows)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    op = SimpleNamespace(shape=A.shape, nrows=rows, rowptr=dev(rowptr.astype(np.int64)), col=dev(cols.astype(np.int64)),
+                         w=dev(w), oidx=dev(oidx.astype(np.int64)))
+    want = y0.copy()
+    want[oidx] += -1.5 * (A @ x)
+    out = dev(y0)
+    Helm3d(device="cuda:0").csr_apply(op, dev(x), out, alpha=-1.5, accumulate=True)
+    assert relerr(out.cpu().numpy(), want) <= 1e-13
+    out = dev(y0)
+    Helm3d(device="cuda:0").csr_apply(op, dev(x), out)
+    want = np.empty_like(y0)
+    want[oidx] = A @ x
+    assert relerr(out.cpu().numpy(), want) <= 1e-13
