@@ -77,10 +77,10 @@ __global__ __launch_bounds__(KB) void prolong_add_kernel(MgAxes T, const cpx<R>*
 
 // yc = scale * P^T rf at coarse points: per (z, y) entry of the transposed
 // lists (uniform over the wave), the x entries of the lane's coarse index
-// from the padded list (WX entries, zero weights past the real ones), so the
-// loads of a coarse point are independent and issued together.  WX = 0: the
-// padded width is read at run time.
-template <typename R, int WX>
+// from the padded list (at most 8 entries, the padded width read at run time),
+// so the loads of a coarse point are independent and issued together.
+constexpr int kGatherWidth = 8;
+template <typename R>
 __global__ __launch_bounds__(KB) void restrict_kernel(MgAxes T, double scale, const cpx<R>* __restrict__ rf,
                                                       cpx<R>* __restrict__ yc)
 {
@@ -90,15 +90,13 @@ __global__ __launch_bounds__(KB) void restrict_kernel(MgAxes T, double scale, co
     if (j >= T.nc[1]) return;
     const int ic = min(i, T.nc[0] - 1);
     const long nfx = T.nf[0], nfxy = long(T.nf[0]) * T.nf[1];
-    const int pw = WX > 0 ? WX : T.ax[0].pw;
-    constexpr int KX = WX > 0 ? WX : 8;
-    int fx[KX];
-    double wxv[KX];
+    const int pw = T.ax[0].pw;
+    int fx[kGatherWidth];
+    double wxv[kGatherWidth];
 #pragma unroll
-    for (int e = 0; e < KX; ++e) {
-        const bool real = WX > 0 || e < pw;
-        fx[e] = real ? T.ax[0].pfi[long(ic) * pw + e] : 0;
-        wxv[e] = real ? T.ax[0].pfw[long(ic) * pw + e] : 0.0;
+    for (int e = 0; e < kGatherWidth; ++e) {
+        fx[e] = e < pw ? T.ax[0].pfi[long(ic) * pw + e] : 0;
+        wxv[e] = e < pw ? T.ax[0].pfw[long(ic) * pw + e] : 0.0;
     }
     double re = 0.0, im = 0.0;
     const int z0 = T.ax[2].rp[k], z1 = T.ax[2].rp[k + 1];
@@ -111,8 +109,8 @@ __global__ __launch_bounds__(KB) void restrict_kernel(MgAxes T, double scale, co
             const double wyz = wz * T.ax[1].fw[ey];
             double sr = 0.0, si = 0.0;
 #pragma unroll
-            for (int e = 0; e < KX; ++e) {
-                if (WX > 0 || e < pw) {
+            for (int e = 0; e < kGatherWidth; ++e) {
+                if (e < pw) {
                     const cpx<R> v = rf[base + fx[e]];
                     sr = fma(wxv[e], double(v.re), sr);
                     si = fma(wxv[e], double(v.im), si);
@@ -212,7 +210,10 @@ hipError_t launch_prolong_add(const MgAxes& T, const cpx<R>* xc, cpx<R>* xf, hip
 template <typename R>
 hipError_t launch_restrict(const MgAxes& T, double scale, const cpx<R>* rf, cpx<R>* yc, hipStream_t s)
 {
-    // grids of a ratio of 2 always fit; the gather takes the ratios beyond about 3
+    // a ratio of 2 always fits the window; the gather takes ratios from about 3.9
+    // along x (a run of 32 coarse points no longer fits) and those along y whose
+    // lists exceed the window's 8 rows; beyond 8 entries along x (ratio 4 and
+    // more) neither does
     if (T.ax[0].run > 0 && T.ax[0].pw <= 8 && T.ax[1].pw <= 8) {
         const dim3 gw((T.nc[0] + T.ax[0].run - 1) / T.ax[0].run, (T.nc[1] + 3) / 4, T.nc[2]);
         if (T.ax[1].pw <= 4)
@@ -223,17 +224,8 @@ hipError_t launch_restrict(const MgAxes& T, double scale, const cpx<R>* rf, cpx<
             hipLaunchKernelGGL((restrict_window_kernel<R, 8>), gw, dim3(KB), 0, s, T, scale, rf, yc);
         return hipGetLastError();
     }
-    const dim3 g = transfer_grid(T.nc);
-    switch (T.ax[0].pw) {
-    case 2: hipLaunchKernelGGL((restrict_kernel<R, 2>), g, dim3(KB), 0, s, T, scale, rf, yc); break;
-    case 3: hipLaunchKernelGGL((restrict_kernel<R, 3>), g, dim3(KB), 0, s, T, scale, rf, yc); break;
-    case 4: hipLaunchKernelGGL((restrict_kernel<R, 4>), g, dim3(KB), 0, s, T, scale, rf, yc); break;
-    case 5: hipLaunchKernelGGL((restrict_kernel<R, 5>), g, dim3(KB), 0, s, T, scale, rf, yc); break;
-    default:
-        if (T.ax[0].pw < 1 || T.ax[0].pw > 8) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((restrict_kernel<R, 0>), g, dim3(KB), 0, s, T, scale, rf, yc);
-        break;
-    }
+    if (T.ax[0].pw < 1 || T.ax[0].pw > kGatherWidth) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(restrict_kernel<R>, transfer_grid(T.nc), dim3(KB), 0, s, T, scale, rf, yc);
     return hipGetLastError();
 }
 

@@ -204,3 +204,36 @@ def test_mg_cycle_lengths(k, precision):
         assert info.converged and np.linalg.norm(r) < 1e-9 * np.linalg.norm(b)
         z, iz = M.solve(torch.zeros_like(x), mode=mode, tol=1e-9, precision=precision)
         assert iz.converged and not z.cpu().numpy().any()
+
+
+# x ratios of 3, 3.5 and 3.65 (windows of 7 and 8 entries), 3.9 (runs below 32
+# points: the gather) and 2 beside a y ratio of 4.5 (y lists beyond the window's
+# 8 rows: the gather); y ratios of 2 to 3.4
+@pytest.mark.parametrize("nf,nc", [((196, 21, 13), (66, 7, 5)), ((229, 13, 15), (66, 7, 5)), ((241, 24, 12), (66, 7, 4)),
+                                   ((255, 20, 13), (66, 7, 5)), ((131, 60, 9), (66, 14, 5))])
+def test_transfer_ratios(nf, nc):
+    """Transfers between grids of any ratio: contexts built one by one, as a
+    caller of helm3d_mg_create may."""
+    import ctypes
+    import torch
+    from helm3d import Helm3d
+    from helm3d._lib import check, lib
+    print("transfer", nf, nc, flush=True)
+    dev = torch.device("cuda:0")
+    op = lambda n: Helm3d(n, (10.0,) * 3, np.full((2, 3), 2),  # noqa: E731
+                          torch.full((int(np.prod(n)),), 1e-4, dtype=torch.float64, device=dev))
+    ops, smoothers = [op(nf), op(nc)], [op(nf), op(nc)]
+    ptrs = lambda hs: (ctypes.c_void_p * 2)(*[h._ctx.value for h in hs])  # noqa: E731
+    mg = ctypes.c_void_p()
+    check(lib().helm3d_mg_create(2, ptrs(ops), ptrs(smoothers), ctypes.byref(mg)))
+    rng = np.random.default_rng(4)
+    P = O.prolongation(nf, nc)
+    xc = rng.standard_normal(P.shape[1]) + 1j * rng.standard_normal(P.shape[1])
+    xf = rng.standard_normal(P.shape[0]) + 1j * rng.standard_normal(P.shape[0])
+    for x, out, d in ((xc, np.zeros(P.shape[0], complex), 0), (xf, np.zeros(P.shape[1], complex), 1)):
+        xt, yt = torch.from_numpy(x).to(dev), torch.from_numpy(out).to(dev)
+        check(lib().helm3d_mg_transfer(mg, 0, d, ctypes.c_void_p(xt.data_ptr()), ctypes.c_void_p(yt.data_ptr())))
+        torch.cuda.synchronize()
+        want = P @ x if d == 0 else (P.T @ x) / 8
+        assert np.linalg.norm(yt.cpu().numpy() - want) <= 1e-13 * np.linalg.norm(want)
+    lib().helm3d_mg_destroy(mg)
