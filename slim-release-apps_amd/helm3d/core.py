@@ -19,10 +19,16 @@ from . import _lib
 from ._lib import check, lib
 
 
+# The raw handle of a device's current stream.  torch.cuda.current_stream()
+# builds a Stream object for it (2.7 us of an 11 us call); this one is not
+# public, so it is used only where it exists.
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_ptr() -> int:
-    # the current stream of the current device (torch.cuda.current_stream()
-    # builds a Stream object for it: 2.7 us of an 11 us call)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _RAW_STREAM is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _RAW_STREAM(torch.cuda.current_device())
 
 
 _SAME_DEVICE = contextlib.nullcontext()
@@ -101,7 +107,7 @@ class Helm3d:
         """torch.cuda.device(self.device), or nothing where that device is
         current already."""
         index = self.device.index
-        if index is not None and index == torch._C._cuda_getDevice():
+        if index is not None and index == torch.cuda.current_device():
             return _SAME_DEVICE
         return torch.cuda.device(self.device)
 
