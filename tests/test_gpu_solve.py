@@ -298,3 +298,64 @@ def test_solve_stops_at_maxit_like_oracle(m, maxit):
     assert np.allclose(info.hst[:k], io["hst"][:k], rtol=1e-8, atol=0)
     x = x.cpu().numpy()
     assert np.linalg.norm(x - xo) / np.linalg.norm(xo) <= 1e-8
+
+
+def _wnc_problem(n, npml, freq, loss):
+    from helm3d.models import config_small, extend, point_source, vec, wavenumber
+    cfg = config_small(n=n, npml=npml, freq=freq, seed=22)
+    wn = vec(wavenumber(extend(cfg.v, cfg.npml), cfg.freq)) * (1.0 + 1j * loss)
+    return cfg, wn, point_source(cfg, cfg.sources[0])
+
+
+def _relres_wnc(cfg, wn, b, x, mode):
+    r = b - O.hmvp("forw_wnc" if mode == 1 else "adj_wnc", wn, (cfg.h,) * 3, cfg.nt, np.array(cfg.npml6), x)
+    return np.linalg.norm(r) / np.linalg.norm(b)
+
+
+# 33 x 31 x 26 points: flexible steps of a short vector (matvec and dots in one
+# launch); 95 x 66 x 58: above their length.  Odd and even numbers of inner
+# iterations end in the one and the other set of the rotating slots.
+@pytest.mark.parametrize("n", [(21, 19, 14), (83, 54, 46)])
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("inner,inner_tol,inner_maxit", [("bicgstab", 0.0, 9), ("bicgstab", 0.0, 10),
+                                                         ("bicgstab", 1e-2, 60), ("gmres", 1e-2, 60)])
+def test_mixed_solve_complex_wavenumber(n, mode, inner, inner_tol, inner_maxit):
+    import torch
+    from helm3d import Helm3d
+    cfg, wn, b = _wnc_problem(n, 6, 5.0, 0.05)
+    print(f"mixed wnc nt={cfg.nt} mode={mode} {inner} {inner_tol} {inner_maxit}", flush=True)
+    dev = torch.device("cuda:0")
+    H = Helm3d(cfg.nt, (cfg.h,) * 3, cfg.npml6, torch.from_numpy(wn).to(dev))
+    x, info = H.solve_mixed(torch.from_numpy(b).to(dev), mode=mode, tol=1e-6, inner=inner, inner_tol=inner_tol,
+                            inner_maxit=inner_maxit)
+    rel = _relres_wnc(cfg, wn, b, x.cpu().numpy(), mode)
+    print("  iters", info.iters, "relres", info.relres, rel, flush=True)
+    assert info.converged and rel < 1e-6 and abs(rel - info.relres) < 1e-9
+
+
+@pytest.mark.parametrize("precision", ["c128", "mixed"])
+@pytest.mark.parametrize("mode", [1, 2])
+def test_multigrid_complex_wavenumber(mode, precision):
+    """A hierarchy whose levels got complex wavenumbers: smoothers and coarse
+    solves run the device-driven steps of short vectors (first step of a solve
+    and of a restarted cycle, norms from partial sums) on the complex-wn
+    operator, in complex128 and complex64."""
+    import torch
+    from helm3d.mg import MLGMRES
+    from helm3d.models import vec
+    cfg, wn, b = _wnc_problem((40, 36, 30), 8, 6.0, 0.05)
+    print(f"mg wnc mode={mode} {precision}", flush=True)
+    M = MLGMRES(vec(cfg.v), cfg.n_phys, cfg.h, cfg.npml, cfg.freq, nlevels=3, k=(2, 3, 2, 5), autotune=False)
+    v = torch.from_numpy(np.ascontiguousarray(vec(cfg.v))).cuda()
+    from helm3d.mg import coarsen_model
+    for lvl, g in enumerate(M.grids):
+        if lvl > 0:
+            v = coarsen_model(v, M.grids[lvl - 1]["n_phys"], g["n_phys"])
+        w = M.ops[lvl].param2wavenum(v, g["n_phys"], g["p6"], cfg.freq, M.unit, derivs=0)[0] * (1.0 + 0.05j)
+        M.ops[lvl].set_model(g["nt"], g["h"], g["p6"], w)
+        M.smoothers[lvl].set_model(g["nt"], g["h"], g["p6"], w)
+    x, info = M.solve(torch.from_numpy(b).cuda(), mode=mode, tol=1e-6, precision=precision)
+    rel = _relres_wnc(cfg, wn, b, x.cpu().numpy(), mode)
+    plain, info_p = M.H.solve(torch.from_numpy(b).cuda(), mode=mode, tol=1e-6)
+    print("  iters", info.iters, "plain", info_p.iters, "relres", info.relres, rel, flush=True)
+    assert info.converged and rel < 1e-6 and info.iters < 0.5 * info_p.iters
