@@ -1,6 +1,6 @@
-// Device body of the 27-point stencil (included by the kernel files).
-//
-// and complex-wavenumber forms in one z-marching kernel template.
+// Device body of the 27-point stencil (included by the kernel files): forward,
+// adjoint, wavenumber-derivative and complex-wavenumber forms in one z-marching
+// kernel template.
 //
 // Reference semantics: do_Hmvp of SLIM-release-apps
 // tools/algorithms/3DFreqModeling/Helm3d_27pt.h:827-875 with the coefficients
@@ -48,10 +48,10 @@ __device__ inline cpx<R> zero() { return cpx<R>{R(0), R(0)}; }
 template <typename T, typename R>
 __device__ inline cpx<T> conv(cpx<R> a) { return cpx<T>{T(a.re), T(a.im)}; }
 
-// Output stores carry the non-temporal hint: no output is read again by the
-// launch that writes it, and streaming the outputs past the caches leaves
-// them to the halo planes of the inputs (the 240x240x140 matvec: 4-7 %
-// faster in FP64 and complex64, forward and adjoint).
+// Output stores carry the non-temporal hint where no output is read again by
+// the launch that writes it (all epilogues but 5): streaming the outputs past
+// the caches leaves them to the halo planes of the inputs (the 240x240x140
+// matvec: 4-7 % faster in FP64 and complex64, forward and adjoint).
 template <typename R>
 __device__ __forceinline__ void st_out(cpx<R>* p, cpx<R> v)
 {
@@ -77,10 +77,11 @@ __device__ inline Cd cd_div(Cd a, Cd b)
     return Cd{fma(a.re, b.re, a.im * b.im) / d, fma(a.im, b.re, -(a.re * b.im)) / d};
 }
 
-// TY: rows of the column tile; RY: rows per thread (1 or 2: a block is
-// 64 x TY / RY threads, one wave per RY consecutive rows, and the 3 x (RY+2)
-// window of a plane is read once for the RY outputs); PF: planes of global
-// loads kept in flight ahead of the plane being computed (1 to 4).
+// TXW, TY: columns and rows of the column tile (a wave is one row of 64 columns
+// or two of 32); RY: rows per thread (1 or 2: a block is TXW x TY / RY threads
+// and the 3 x (RY+2) window of a plane is read once for the RY outputs); PF:
+// planes of global loads kept in flight ahead of the plane being computed (1 to
+// 4).
 //
 // Memory pipeline: every global load of the loop goes into one of PF register
 // sets that are refilled right after being staged into LDS, so no register is
@@ -183,8 +184,9 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
     // plane's 3x3 neighbourhood (24 registers instead of 18 complex
     // coefficients).  Adjoint: side values of the neighbours, conjugated.
     // Forward, the face multipliers are the sums of the side ones and are not
-    // formed.  The y multipliers are uniform over the wave (rows jw ..
-    // jw+RY-1): read at wave-uniform indices so they live in scalar registers.
+    // formed.  In a 64-column tile the y multipliers are uniform over the wave
+    // (rows jw .. jw+RY-1) and live in scalar registers; a wave of a 32-column
+    // tile is two rows and holds them per lane.
     cpx<R> px0{}, px2{}, pxf{};
     cpx<R> py0[RY], py2[RY], pyf[RY];
     if constexpr (!DERIV) {
@@ -640,7 +642,10 @@ __device__ __forceinline__ void helm27_body(const StencilLaunch<R>& L, const int
                 cpx<R> res = alpha * out;
                 if constexpr (EPI == 1) res = rfma(res, L.beta, bb[r]);
                 cpx<R>* dst = live ? &L.y[long(kc) * plane + offc[r]] : &L.sink[sk];
-                st_out(dst, res);
+                // EPI 5 reads y back for its dots: kept in the caches (multigrid
+                // solves 1 % faster than with the hint)
+                if constexpr (EPI == 5) *dst = res;
+                else st_out(dst, res);
                 if (live) acc[0] += double(res.re) * double(res.re) + double(res.im) * double(res.im);
             }
         }
