@@ -155,14 +155,17 @@ bool narrow_tiles(int nx)
 // item's partial sums follow its chunk, so the chunk must not depend on what
 // else is in the batch and has to do for one item as for thirty.  The cost model
 // is asked for a launch of four such items, with two exceptions:
-// * below 32 tiles no more than 8 planes: 84 x 72 x 50, two outer steps of 1 / 4
-//   / 16 items: 14 planes 2.39 / 3.32 / 9.17 ms, 8 planes 1.88 / 3.05 / 9.10;
+// * below 30 tiles no more than 10 planes: 84 x 72 x 50, two outer steps of 1 /
+//   4 / 16 items: 14 planes 2.3 / 3.2 / 9.1 ms, 10 planes 1.95 / 3.2 / 9.0, 8
+//   planes 1.85 / 3.0 / 9.0; but 72 x 64 x 60 of 4 / 8 items: 12 planes 3.0 / 4.7,
+//   10 planes 3.2 / 5.1, 8 planes 3.0 / 5.2;
 // * from 240 to 479 tiles, where one item in two chunks fills the chip, two
 //   chunks: 240 x 240 x 140 x 8: 48 planes 78.2 ms, 70 planes 75.8.
 // Elsewhere the model weighs few items against many: against about 480 blocks
-// an item it gains 9 % on 120 x 90 x 60 x 8 (8.4 ms, 9.2) and 20 % on one or two
-// 48 x 48 x 40 items (1.40, 1.75), and loses 8 % on one 128 x 128 x 80 item (3.1,
-// 2.8) and 14 % on sixteen 48 x 48 x 40 ones (4.3, 3.75).
+// an item it gains 9 % on 120 x 90 x 60 x 8 (8.4 ms, 9.2), 17 % on 94 x 73 x 63 x
+// 2 to 8 and 20 % on one or two 48 x 48 x 40 items (1.40, 1.75), and loses 8 % on
+// one 128 x 128 x 80 item (3.1, 2.8), 12 % on one of 94 x 73 x 63 and 14 % on
+// sixteen of 48 x 48 x 40 (4.3, 3.75).
 StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, int ry, bool mix)
 {
     if (mix) {
@@ -176,7 +179,7 @@ StencilGrid item_grid(const helm3d_ctx* c, int ty, int pf, int ry, bool mix)
         const StencilGrid g = stencil_grid<double>(c->n[0], c->n[1], c->n[2], 1, ty, pf, ry, tx);
         const int tiles = g.tiles_x * g.tiles_y, nz = c->n[2];
         kc = stencil_chunk(4L * tiles, nz, kCost64);
-        if (tiles < 32) kc = std::min(kc, 8);
+        if (tiles < 30) kc = std::min(kc, 10);
         else if (tiles >= 240 && tiles < 480) kc = (nz + 1) / 2;
     }
     return stencil_grid<double>(c->n[0], c->n[1], c->n[2], kc, ty, pf, ry, tx);
