@@ -151,6 +151,8 @@ struct helm3d_ctx {
     StencilGrid rule64{}, rule32{};
     // the fused BiCGStab forms of a single mixed solve, by rule as well
     StencilGrid fused{};
+    // the wavenumber-derivative forms while no shape is chosen
+    StencilGrid deriv64{}, deriv32{};
 
     double* part = nullptr;
     size_t part_cap = 0;
@@ -277,6 +279,13 @@ inline const StencilGrid& grid_of(const helm3d_ctx* c)
 {
     if constexpr (std::is_same<R, double>::value) return c->grid;
     else return c->grid32;
+}
+template <typename R>
+inline const StencilGrid& deriv_of(const helm3d_ctx* c)
+{
+    if (!c->grid_auto) return grid_of<R>(c);
+    if constexpr (std::is_same<R, double>::value) return c->deriv64;
+    else return c->deriv32;
 }
 template <typename R>
 inline const StencilGrid& rule_of(const helm3d_ctx* c)

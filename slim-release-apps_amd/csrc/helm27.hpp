@@ -120,6 +120,16 @@ int stencil_chunk(long tiles, int nz, const ChunkCost& m);
 template <typename R>
 StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 8, int pf = 2, int ry = 1, int tx = 0);
 
+// The shape by rule of the wavenumber-derivative forms (gradient epilogue among
+// them).  They hold no PML sums and wait for memory, so grids of more than 100
+// column tiles take few long chunks, about 480 blocks in all: derivative matvec
+// in complex128 forward / adjoint and gradient on 240 x 240 x 140 with the chunk
+// of the operator 72.7 / 63.4 and 90.5 us, so 67.0 / 58.0 and 83.4; 296 x 296 x
+// 168 in complex64 126.9 / 118.3, so 114.7 / 107.7.  Smaller grids keep the
+// operator's chunk (120 x 110 x 90: 10.9 us with 10 planes, 11.4 with 12).
+template <typename R>
+StencilGrid stencil_deriv_grid(int nx, int ny, int nz);
+
 template <typename R>
 hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g, hipStream_t s);
 

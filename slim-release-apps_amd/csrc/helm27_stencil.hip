@@ -144,6 +144,18 @@ hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g,
     return launch_epi<R, true, true, true>(L, g, s);
 }
 
+template <typename R>
+StencilGrid stencil_deriv_grid(int nx, int ny, int nz)
+{
+    const StencilGrid g = stencil_grid<R>(nx, ny, nz, 0);
+    const int tiles = g.tiles_x * g.tiles_y;
+    if (tiles <= kLargeTiles) return g;
+    const int chunks = (480 + tiles - 1) / tiles;
+    return stencil_grid<R>(nx, ny, nz, (nz + chunks - 1) / chunks);
+}
+
+template StencilGrid stencil_deriv_grid<double>(int, int, int);
+template StencilGrid stencil_deriv_grid<float>(int, int, int);
 template StencilGrid stencil_grid<double>(int, int, int, int, int, int, int, int);
 template StencilGrid stencil_grid<float>(int, int, int, int, int, int, int, int);
 template hipError_t launch_stencil<double>(int, StencilLaunch<double>, const StencilGrid&, hipStream_t);

@@ -884,6 +884,8 @@ int helm3d_set_model(helm3d_ctx* c, const int n[3], const double h[3], const int
     if (!same_grid) {
         c->grid = c->rule64 = stencil_grid<double>(n[0], n[1], n[2], 0);
         c->grid32 = c->rule32 = stencil_grid<float>(n[0], n[1], n[2], 0);
+        c->deriv64 = stencil_deriv_grid<double>(n[0], n[1], n[2]);
+        c->deriv32 = stencil_deriv_grid<float>(n[0], n[1], n[2]);
         // the fused forms hold two to four vectors a point and fit a compute
         // unit as often as the complex128 kernel: its cost model (97 x 79 x 65:
         // 34.8 ms a solve, 36.6 with the chunk of the plain complex64 kernel);
@@ -1049,14 +1051,14 @@ int helm3d_apply_deriv(helm3d_ctx* c, int adjoint, int precision, const void* dw
         op.wn = static_cast<const double*>(dwn);
         op.wnc = nullptr;
         return stencil<double>(c, v, op, static_cast<const cpx<double>*>(x), static_cast<cpx<double>*>(y), 1.0,
-                               nullptr, 0.0, nullptr);
+                               nullptr, 0.0, nullptr, nullptr, &deriv_of<double>(c));
     }
     if (precision == HELM3D_C64) {
         OpDesc<float> op = c->op32;
         op.wn = static_cast<const float*>(dwn);
         op.wnc = nullptr;
         return stencil<float>(c, v, op, static_cast<const cpx<float>*>(x), static_cast<cpx<float>*>(y), 1.0f,
-                              nullptr, 0.0f, nullptr);
+                              nullptr, 0.0f, nullptr, nullptr, &deriv_of<float>(c));
     }
     return fail(HELM3D_ERR_ARG, "bad precision");
 }
@@ -1191,7 +1193,7 @@ int helm3d_fwi_grad_accum(helm3d_ctx* c, const double* dwn, const void* U, const
         L.pn[a] = phys ? c->n[a] - c->npml[2 * a] - c->npml[2 * a + 1] : c->n[a];
         if (L.pn[a] < 1) return fail(HELM3D_ERR_ARG, "PML covers the whole axis");
     }
-    HIPCHK(launch_stencil<double>(VAR_ADJ | VAR_DERIV, L, c->grid, c->stream));
+    HIPCHK(launch_stencil<double>(VAR_ADJ | VAR_DERIV, L, deriv_of<double>(c), c->stream));
     return HELM3D_OK;
 }
 

@@ -147,8 +147,9 @@ int helm3d_apply_noalloc(int variant, const int n[3], const double h[3], const i
     L.alpha = 1.0;
     L.beta = 0.0;
     L.sink = sink;
-    const StencilGrid g = stencil_grid<double>(n[0], n[1], n[2], 0);
     const int v = variant | (wn_complex ? VAR_WNC : 0);
+    const StencilGrid g = (v & VAR_DERIV) ? stencil_deriv_grid<double>(n[0], n[1], n[2])
+                                          : stencil_grid<double>(n[0], n[1], n[2], 0);
     HIPCHK(launch_stencil<double>(v, L, g, s));
     return HELM3D_OK;
 }
