@@ -151,8 +151,9 @@ struct helm3d_ctx {
     StencilGrid rule64{}, rule32{};
     // the fused BiCGStab forms of a single mixed solve, by rule as well
     StencilGrid fused{};
-    // the wavenumber-derivative forms while no shape is chosen
-    StencilGrid deriv64{}, deriv32{};
+    // the wavenumber-derivative forms and the complex128 residual while no shape
+    // is chosen
+    StencilGrid deriv64{}, deriv32{}, resid64{};
 
     double* part = nullptr;
     size_t part_cap = 0;
@@ -288,6 +289,12 @@ inline const StencilGrid& deriv_of(const helm3d_ctx* c)
     else return c->deriv32;
 }
 template <typename R>
+inline const StencilGrid& resid_of(const helm3d_ctx* c)
+{
+    if constexpr (std::is_same<R, double>::value) return c->grid_auto ? c->resid64 : c->grid;
+    else return c->grid32;
+}
+template <typename R>
 inline const StencilGrid& rule_of(const helm3d_ctx* c)
 {
     if constexpr (std::is_same<R, double>::value) return c->rule64;
@@ -347,7 +354,8 @@ constexpr long kMaxDeviceCycles = 16;
 inline int ensure_work(helm3d_ctx* c)
 {
     const size_t nblk = std::max<size_t>({size_t(kMaxPartials), size_t(c->grid.blocks), size_t(c->grid32.blocks),
-                                          size_t(c->rule64.blocks), size_t(c->rule32.blocks), size_t(c->fused.blocks)});
+                                          size_t(c->rule64.blocks), size_t(c->rule32.blocks), size_t(c->fused.blocks),
+                                          size_t(c->resid64.blocks)});
     CHK(ensure_t(&c->part, &c->part_cap, nblk * 2 * kMaxBasis));
     CHK(ensure_t(&c->small, &c->small_cap, 2 * kMaxBasis + 8));
     CHK(ensure(&c->sink, &c->sink_cap, size_t(kSinkSlots) * sizeof(cpx<double>)));

@@ -105,7 +105,8 @@ struct ChunkCost {
     int slots;
     double halo, fill, wait, tail;
 };
-constexpr ChunkCost kCost64{512, 2, 2, 0.2, 0.15}, kCost64Large{768, 4, 0, 0.15, 0.15}, kCost32{1024, 2, 2, 0.2, 0.15};
+constexpr ChunkCost kCost64{512, 2, 2, 0.2, 0.15}, kCost64Large{768, 4, 0, 0.15, 0.15}, kCost64Resid{512, 1, 2, 0, 0.25},
+    kCost32{1024, 2, 2, 0.2, 0.15};
 constexpr int kLargeTiles = 100;
 int stencil_chunk(long tiles, int nz, const ChunkCost& m);
 
@@ -129,6 +130,14 @@ StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 8, int pf 
 // operator's chunk (120 x 110 x 90: 10.9 us with 10 planes, 11.4 with 12).
 template <typename R>
 StencilGrid stencil_deriv_grid(int nx, int ny, int nz);
+
+// The shape by rule of the complex128 residual form (b - H x).  With the addend
+// in flight two blocks fit a compute unit and an uneven last round costs more;
+// its constants find the best chunk of the sweep on eight grids of 84^3 to 280 x
+// 280 x 140.  They are used from the size at which the operator's differ (240 x
+// 240 x 140: 48 planes 115.8 us, 70 planes 93.9; 187 x 203 x 111: 28 planes 61.5,
+// 37 planes 50.9; 64 x 4 tiles in 480 blocks 98.2 and 57.2).
+StencilGrid stencil_resid_grid(int nx, int ny, int nz);
 
 template <typename R>
 hipError_t launch_stencil(int variant, StencilLaunch<R> L, const StencilGrid& g, hipStream_t s);

@@ -154,6 +154,13 @@ StencilGrid stencil_deriv_grid(int nx, int ny, int nz)
     return stencil_grid<R>(nx, ny, nz, (nz + chunks - 1) / chunks);
 }
 
+StencilGrid stencil_resid_grid(int nx, int ny, int nz)
+{
+    const StencilGrid g = stencil_grid<double>(nx, ny, nz, 0);
+    const int tiles = g.tiles_x * g.tiles_y;
+    return tiles <= kLargeTiles ? g : stencil_grid<double>(nx, ny, nz, stencil_chunk(tiles, nz, kCost64Resid));
+}
+
 template StencilGrid stencil_deriv_grid<double>(int, int, int);
 template StencilGrid stencil_deriv_grid<float>(int, int, int);
 template StencilGrid stencil_grid<double>(int, int, int, int, int, int, int, int);

@@ -290,8 +290,9 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
     // r0 = b - A x0, or b with x = 0 (FGMRES.m:57-62); ||r0||^2 into nrm[0]
     // and the pinned mirror
     if (use_x0) {
-        CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part));
-        TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, grid_of<R>(c).blocks, 1, c->nrm, c->stream, c->small_host_dev));
+        CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, nullptr, &resid_of<R>(c)));
+        TIMED(HELM3D_PROF_REDUCE,
+              launch_reduce(c->part, resid_of<R>(c).blocks, 1, c->nrm, c->stream, c->small_host_dev));
     } else {
         HIPCHK(launch_start<R>(b, slot(0), x, N, c->part, nblk, c->stream));
         TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, nblk, 1, c->nrm, c->stream, c->small_host_dev));
@@ -356,8 +357,9 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
         for (long cyc = 0; (1 + cyc * long(m)) / m < maxit; ++cyc) {
             if (cyc > 0) {
                 HIPCHK(launch_gmres_gate(st, c->stream));
-                CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, skip));
-                TIMED(HELM3D_PROF_REDUCE, launch_reduce(c->part, grid_of<R>(c).blocks, 1, c->nrm, c->stream, nullptr, skip));
+                CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, skip, &resid_of<R>(c)));
+                TIMED(HELM3D_PROF_REDUCE,
+                      launch_reduce(c->part, resid_of<R>(c).blocks, 1, c->nrm, c->stream, nullptr, skip));
                 HIPCHK(launch_gmres_restart(c->nrm, tol, st, c->stream));
             }
             CHK(enqueue_cycle(use_graph));
@@ -518,8 +520,8 @@ int gmres_engine(helm3d_ctx* c, int variant, const cpx<R>* b, cpx<R>* x, bool us
             break;
         }
         // true residual r = b - A x into slot 0, FGMRES.m:120-124
-        CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part));
-        CHK(reduce_to_small(c, grid_of<R>(c).blocks, 1, 0, c->nrm));
+        CHK(stencil<R>(c, variant, op, x, slot(0), R(-1), b, R(1), c->part, nullptr, &resid_of<R>(c)));
+        CHK(reduce_to_small(c, resid_of<R>(c).blocks, 1, 0, c->nrm));
         CHK(fetch_small(c, 1));
         const double rn = std::sqrt(c->small_host[0]);
         res->relres = rn / normr0;
@@ -886,6 +888,7 @@ int helm3d_set_model(helm3d_ctx* c, const int n[3], const double h[3], const int
         c->grid32 = c->rule32 = stencil_grid<float>(n[0], n[1], n[2], 0);
         c->deriv64 = stencil_deriv_grid<double>(n[0], n[1], n[2]);
         c->deriv32 = stencil_deriv_grid<float>(n[0], n[1], n[2]);
+        c->resid64 = stencil_resid_grid(n[0], n[1], n[2]);
         // the fused forms hold two to four vectors a point and fit a compute
         // unit as often as the complex128 kernel: its cost model (97 x 79 x 65:
         // 34.8 ms a solve, 36.6 with the chunk of the plain complex64 kernel);
@@ -1092,8 +1095,8 @@ int helm3d_solve_bicgstab(helm3d_ctx* c, int mode, const void* b, void* x, const
     CHK(bicgstab_engine<double>(c, variant, bb, xx, o.tol, long(o.maxit), 1, &its, &rel));
     // true residual ||b - A x|| / ||b|| in FP64
     CHK(ensure_vecs(c->T64, c->N, 1));
-    CHK(stencil<double>(c, variant, c->op64, xx, c->T64.p, -1.0, bb, 1.0, c->part));
-    CHK(reduce_to_small(c, c->grid.blocks, 1, 0));
+    CHK(stencil<double>(c, variant, c->op64, xx, c->T64.p, -1.0, bb, 1.0, c->part, nullptr, &resid_of<double>(c)));
+    CHK(reduce_to_small(c, resid_of<double>(c).blocks, 1, 0));
     HIPCHK(launch_norm2<double>(bb, c->N, c->part, krylov_blocks(c->N), c->stream));
     CHK(reduce_to_small(c, krylov_blocks(c->N), 1, 1));
     CHK(fetch_small(c, 2));

@@ -50,8 +50,9 @@ int finish_kacz_solve(helm3d_ctx* c, int mode, const cpx<double>* b, const cpx<d
     L.beta = 1.0;
     L.norm_part = c->part;
     L.sink = static_cast<cpx<double>*>(c->sink);
-    HIPCHK(launch_stencil<double>((mode != 1 ? VAR_ADJ : VAR_FORW) | (c->wnc ? VAR_WNC : 0), L, c->grid, st));
-    HIPCHK(launch_reduce(c->part, c->grid.blocks, 1, c->small, st));
+    const StencilGrid& G = resid_of<double>(c);
+    HIPCHK(launch_stencil<double>((mode != 1 ? VAR_ADJ : VAR_FORW) | (c->wnc ? VAR_WNC : 0), L, G, st));
+    HIPCHK(launch_reduce(c->part, G.blocks, 1, c->small, st));
     HIPCHK(launch_norm2<double>(b, N, c->part, nblk, st));
     HIPCHK(launch_reduce(c->part, nblk, 1, c->small + 1, st));
     HIPCHK(hipMemcpyAsync(c->small_host, c->small, 2 * sizeof(double), hipMemcpyDeviceToHost, st));

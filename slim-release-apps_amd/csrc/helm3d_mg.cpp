@@ -206,7 +206,7 @@ int residual(MgLevel& L, int mode, const cpx<R>* b, const cpx<R>* x, cpx<R>* r)
     S.alpha = R(-1);
     S.beta = R(1);
     S.sink = static_cast<cpx<R>*>(L.A->sink);
-    HIPCHK(launch_stencil<R>(model_variant(L.A, mode != 1), S, grid_of<R>(L.A), L.A->stream));
+    HIPCHK(launch_stencil<R>(model_variant(L.A, mode != 1), S, resid_of<R>(L.A), L.A->stream));
     return HELM3D_OK;
 }
 
