@@ -737,8 +737,8 @@ def main():
     for r in (roofline, stencil_roofline):
         r["measured_copy_GBps"] = copy_gbs
         r["frac_of_measured_copy"] = r["achieved"] / copy_gbs
-    stencil_roofline["note"] = ("near the FP64 vector ridge (78.6 TFLOP/s / 8 TB/s = 10 flop/B): about 173 VALU "
-                                "instructions (mostly FP64) and 22 LDS instructions per point against 40 B; the "
+    stencil_roofline["note"] = ("near the FP64 vector ridge (78.6 TFLOP/s / 8 TB/s = 10 flop/B): about 164 VALU "
+                                "instructions (mostly FP64) and 21 LDS instructions per point against 40 B; the "
                                 "arithmetic does not fully overlap memory (a copy of the kernel without it runs at "
                                 "4.8-5.3 TB/s), and more planes of loads in flight cost registers")
     for v in breakdown.values():

@@ -115,9 +115,11 @@ int stencil_chunk(long tiles, int nz, const ChunkCost& m);
 // of 32 columns, of 64 with two rows per thread.  Tiles of 32 x 8 read 1.33
 // points per output and waste no more than 31 lanes of a row, tiles of 64 x 4
 // with the same threads 1.55 and 63; and more waves lie outside the PML.
-// Against 64 x 4, complex128 forward / complex64 adjoint: 84^3 14.9 -> 12.6 /
-// 11.7 -> 9.6 us, 160 x 160 x 80 28.0 -> 23.9 / 18.9 -> 16.1, 240 x 240 x 140
-// 93.9 -> 85.9 / 54.7 -> 47.8, 280 x 280 x 140 119 -> 105 / 71.2 -> 61.5.
+// Against 64 x 4 in about 480 blocks, both with the chunk by their rule,
+// complex128 / complex64 forward on rotating inputs: 84^3 14.4 -> 11.9 / 11.1 ->
+// 9.9 us, 160 x 160 x 80 26.1 -> 21.8 / 20.0 -> 15.7, 240 x 240 x 140 82.5 -> 79.7 /
+// 59.7 -> 50.7, 280 x 280 x 140 108 -> 95 / 69.9 -> 61.4; 250 x 100 x 60 19.7 ->
+// 21.3 (100 tiles of 64 x 4 made 500 equal blocks).
 template <typename R>
 StencilGrid stencil_grid(int nx, int ny, int nz, int kchunk, int ty = 8, int pf = 2, int ry = 1, int tx = 0);
 
